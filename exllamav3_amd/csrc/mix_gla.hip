@@ -475,12 +475,39 @@ __global__ __launch_bounds__(256) void gla_chunk_kernel(float* __restrict__ o, c
             f4 A = *(const f4*) (ap + r16 * 20 + 4 * g), P[2] = { f4{ 0.f, 0.f, 0.f, 0.f }, f4{ 0.f, 0.f, 0.f, 0.f } };
             #pragma unroll
             for (int u = 1; u < 4; ++u) A += *(const f4*) (ap + (u * 16 + r16) * 20 + 4 * g);
+            // A row of v that is not finite must not reach the rows in front of it, whose entries of A are zero (0 times infinity is NaN): such an entry counts as zero in the
+            // product, and its column is NaN from its own row on
+            int bad[2] = { 16, 16 };
+            bool odd = false;
+            #pragma unroll
+            for (int c = 0; c < 2; ++c)
+                #pragma unroll
+                for (int j = 0; j < 4; ++j) odd |= !(fabsf(vv[c][j]) < INFINITY);
+            const bool any_odd = __any(odd);
+            if (any_odd)
+            {
+                #pragma unroll
+                for (int c = 0; c < 2; ++c)
+                {
+                    #pragma unroll
+                    for (int j = 3; j >= 0; --j) if (!(fabsf(vv[c][j]) < INFINITY)) { bad[c] = 4 * g + j; vv[c][j] = 0.f; }
+                    bad[c] = min(bad[c], __shfl_xor(bad[c], 16, 64));
+                    bad[c] = min(bad[c], __shfl_xor(bad[c], 32, 64));
+                }
+            }
             #pragma unroll
             for (int j = 0; j < 4; ++j)
                 #pragma unroll
                 for (int c = 0; c < 2; ++c) P[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[j], vv[c][j], P[c], 0, 0, 0);
             #pragma unroll
             for (int c = 0; c < 2; ++c) P[c] += (O[0][c] + O[1][c]) + (O[2][c] + O[3][c]);
+            if (any_odd)
+            {
+                #pragma unroll
+                for (int c = 0; c < 2; ++c)
+                    #pragma unroll
+                    for (int i = 0; i < 4; ++i) if (4 * g + i >= bad[c]) P[c][i] = NAN;
+            }
             #pragma unroll
             for (int c = 0; c < 2; ++c)
                 #pragma unroll

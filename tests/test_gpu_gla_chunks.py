@@ -50,3 +50,38 @@ def test_segments_match_the_recurrence(H, d, dv, tau, rank, bias, lens, dtype):
         for b in range(B):
             assert float((state[slots[b]] - end[b]).abs().max() / end[b].abs().max()) < 2e-5, L
         assert torch.equal(state[0], start[0])                            # a slot of no sequence stays
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("what", ["v", "k", "q", "lr"])
+def test_a_value_that_is_not_finite_stays_out_of_the_rows_before_it(what, value):
+    """One such element in the middle of a chunk: rows in front of it, the other sequence and (an element of v) the other columns keep their bits; its own row is not finite."""
+    from exllamav3_amd import mix_ops
+    H, d, dv, rank, lens, at, col = 2, 64, 140, 4, [50, 70], 50 + 22, 133                # row 22 of the second sequence: the seventh of its second chunk
+    gen = torch.Generator(device=DEV).manual_seed(3)
+    rnd = lambda *s: torch.randn(*s, device=DEV, generator=gen)
+    N = sum(lens)
+    t = {"q": rnd(N, H * d), "k": rnd(N, H * d), "v": rnd(N, H * dv), "lr": rnd(N, rank)}
+    a2, a2b = rnd(H * d, rank), rnd(H * d) + 1.0
+    mk = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+
+    def scan():
+        state, o = torch.zeros((2, H, d, dv), device=DEV), torch.full((N, H, dv), float("nan"), device=DEV)
+        mix_ops.gla_scan(o, state, t["q"], t["k"], t["v"], t["lr"], a2, a2b, mk([0, 50, 120]), mk([0, 1]), mk([0, 0]), 4.0, 0.125, segments=(2, 48))
+        return o, state
+    plain, _ = scan()
+    assert plain.isfinite().all()
+    t[what][at, {"v": dv + col, "k": 5, "q": 5, "lr": 0}[what]] = value
+    o, state = scan()
+    assert torch.equal(o[:at], plain[:at]) and state[0].isfinite().all()
+    if what == "v":
+        keep = torch.ones((H, dv), dtype=torch.bool, device=DEV)
+        keep[1, col] = False
+        assert torch.equal(o[:, keep], plain[:, keep])
+        assert not o[at:, 1, col].isfinite().any() and not state[1, 1, :, col].isfinite().any()
+    elif what == "q":
+        assert torch.equal(o[at + 1:], plain[at + 1:]) and not o[at, 0].isfinite().any()
+    elif what == "k" or value != value:
+        assert not o[at:, 0].isfinite().any()
+    else:                                                                               # (decays of an infinite input are 0 or 1)
+        assert o.isfinite().all()
