@@ -545,7 +545,7 @@ static int gla_chunk_launch(float* o, const void* q, int64_t q_ld, const void* k
                                              (const T*) lr, lr_ld, (const T*) a2, a2_bias, cu, heads, vdim, rank, 1.0f / tau, q_scale, segs, seg_len, seg_state, seg_decay, decay)
     MIX_DISPATCH_T(dtype, if (dim == 64) { GLA_CHUNK(64); } else { GLA_CHUNK(128); });
     #undef GLA_CHUNK
-    return mix_check_launch("mix_gla_segmented (chunks)");
+    return mix_check_launch("mix_gla_chunked");
 }
 
 template <int MODEV>
@@ -579,30 +579,45 @@ extern "C" int exl3_mix_gla_scan(float* o, float* state, const void* q, int64_t 
                                  1, 0, nullptr, nullptr);
 }
 
-extern "C" int exl3_mix_gla_segmented(float* o, float* state, const void* q, int64_t q_ld, const void* k, int64_t k_ld, const void* v, int64_t v_ld,
-                                      const void* lr, int64_t lr_ld, const void* a2, const float* a2_bias, const int32_t* cu, const int32_t* slots, const int32_t* pos0,
-                                      int batch, int heads, int dim, int vdim, int rank, float tau, float q_scale, int segs, int seg_len,
-                                      float* seg_state, float* seg_decay, float* decay, int dtype, void* stream)
+static int gla_combine_launch(float* state, float* seg_state, const float* seg_decay, const int32_t* cu, const int32_t* slots, const int32_t* pos0, int batch, int heads, int dim, int vdim,
+                              int segs, int seg_len, void* stream)
 {
-    MIX_CHECK(segs >= 1 && seg_len >= 1 && seg_state && seg_decay, "mix_gla_segmented: bad segment arguments");
-    // the chunk form wins from the first segment on (its shapes: key dimensions that are whole matrix tiles of one or two values per lane, a low-rank input that fits LDS)
-    const bool chunks = (dim == 64 || dim == 128) && rank <= GC_MAX_RANK && decay;
-    MIX_CHECK(!chunks || (o && state && q && k && v && lr && a2 && cu && slots && pos0 && batch >= 0 && heads > 0 && vdim > 0 && rank > 0 && tau > 0.f), "mix_gla_segmented: null pointer or sizes out of range");
-    MIX_CHECK(!chunks || (q_ld >= (int64_t) heads * dim && k_ld >= (int64_t) heads * dim && v_ld >= (int64_t) heads * vdim && lr_ld >= rank), "mix_gla_segmented: bad row strides");
-    if (chunks && batch == 0) return EXL3_MIX_OK;
-    int rc = chunks ? gla_chunk_launch<true>(o, q, q_ld, k, k_ld, v, v_ld, lr, lr_ld, a2, a2_bias, cu, batch, heads, dim, vdim, rank, tau, q_scale, dtype, stream, segs, seg_len,
-                                             seg_state, seg_decay, decay)
-                    : gla_launch<GLA_SEG_LOCAL>(o, state, q, q_ld, k, k_ld, v, v_ld, lr, lr_ld, a2, a2_bias, cu, slots, pos0, batch, heads, dim, vdim, rank, tau, q_scale, dtype,
-                                                stream, segs, seg_len, seg_state, seg_decay);
-    if (rc || batch == 0) return rc;
     const int64_t per = (int64_t) dim * vdim;
     hipLaunchKernelGGL(gla_combine_kernel, dim3(batch, heads, (unsigned) ((per + 1023) / 1024)), dim3(256), 0, (hipStream_t) stream, state, seg_state, seg_decay, cu, slots, pos0,
                        heads, dim, vdim, segs, seg_len);
-    if ((rc = mix_check_launch("mix_gla_segmented (combine)"))) return rc;
-    if (chunks) return gla_chunk_launch<false>(o, q, q_ld, k, k_ld, v, v_ld, lr, lr_ld, a2, a2_bias, cu, batch, heads, dim, vdim, rank, tau, q_scale, dtype, stream, segs, seg_len,
-                                               seg_state, seg_decay, decay);
+    return mix_check_launch("mix_gla (combine)");
+}
+
+extern "C" int exl3_mix_gla_segmented(float* o, float* state, const void* q, int64_t q_ld, const void* k, int64_t k_ld, const void* v, int64_t v_ld,
+                                      const void* lr, int64_t lr_ld, const void* a2, const float* a2_bias, const int32_t* cu, const int32_t* slots, const int32_t* pos0,
+                                      int batch, int heads, int dim, int vdim, int rank, float tau, float q_scale, int segs, int seg_len,
+                                      float* seg_state, float* seg_decay, int dtype, void* stream)
+{
+    MIX_CHECK(segs >= 1 && seg_len >= 1 && seg_state && seg_decay, "mix_gla_segmented: bad segment arguments");
+    int rc = gla_launch<GLA_SEG_LOCAL>(o, state, q, q_ld, k, k_ld, v, v_ld, lr, lr_ld, a2, a2_bias, cu, slots, pos0, batch, heads, dim, vdim, rank, tau, q_scale, dtype,
+                                       stream, segs, seg_len, seg_state, seg_decay);
+    if (rc || batch == 0) return rc;
+    if ((rc = gla_combine_launch(state, seg_state, seg_decay, cu, slots, pos0, batch, heads, dim, vdim, segs, seg_len, stream))) return rc;
     return gla_launch<GLA_SEG_FINAL>(o, state, q, q_ld, k, k_ld, v, v_ld, lr, lr_ld, a2, a2_bias, cu, slots, pos0, batch, heads, dim, vdim, rank, tau, q_scale, dtype,
                                      stream, segs, seg_len, seg_state, seg_decay);
+}
+
+// its shapes: key dimensions that are whole matrix tiles of one or two values per lane, a low-rank input that fits LDS; there the chunk form wins from the first segment on
+extern "C" int exl3_mix_gla_chunked(float* o, float* state, const void* q, int64_t q_ld, const void* k, int64_t k_ld, const void* v, int64_t v_ld,
+                                    const void* lr, int64_t lr_ld, const void* a2, const float* a2_bias, const int32_t* cu, const int32_t* slots, const int32_t* pos0,
+                                    int batch, int heads, int dim, int vdim, int rank, float tau, float q_scale, int segs, int seg_len,
+                                    float* seg_state, float* seg_decay, float* decay, int dtype, void* stream)
+{
+    MIX_CHECK(segs >= 1 && seg_len >= 1 && seg_state && seg_decay && decay, "mix_gla_chunked: bad segment arguments");
+    MIX_CHECK((dim == 64 || dim == 128) && rank <= GC_MAX_RANK, "mix_gla_chunked: key dimension 64 or 128, rank at most %d", GC_MAX_RANK);
+    MIX_CHECK(o && state && q && k && v && lr && a2 && cu && slots && pos0 && batch >= 0 && heads > 0 && vdim > 0 && rank > 0 && tau > 0.f, "mix_gla_chunked: null pointer or sizes out of range");
+    MIX_CHECK(q_ld >= (int64_t) heads * dim && k_ld >= (int64_t) heads * dim && v_ld >= (int64_t) heads * vdim && lr_ld >= rank, "mix_gla_chunked: bad row strides");
+    if (batch == 0) return EXL3_MIX_OK;
+    int rc = gla_chunk_launch<true>(o, q, q_ld, k, k_ld, v, v_ld, lr, lr_ld, a2, a2_bias, cu, batch, heads, dim, vdim, rank, tau, q_scale, dtype, stream, segs, seg_len,
+                                    seg_state, seg_decay, decay);
+    if (rc || (rc = gla_combine_launch(state, seg_state, seg_decay, cu, slots, pos0, batch, heads, dim, vdim, segs, seg_len, stream))) return rc;
+    return gla_chunk_launch<false>(o, q, q_ld, k, k_ld, v, v_ld, lr, lr_ld, a2, a2_bias, cu, batch, heads, dim, vdim, rank, tau, q_scale, dtype, stream, segs, seg_len,
+                                   seg_state, seg_decay, decay);
 }
 
 extern "C" int exl3_mix_gla_out(void* out, const float* o, const float* w, const void* g, int64_t g_ld, float eps, int n, int heads, int vdim, int dtype, void* stream)

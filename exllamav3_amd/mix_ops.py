@@ -158,8 +158,12 @@ def gla_scan(o, state, q_view, k_view, v_view, lr_view, a2, a2_bias, cu, slots, 
     segs, seg_len = segments
     seg_state = torch.empty((batch * segs, heads, dim, vdim), dtype=torch.float32, device=o.device)
     seg_decay = torch.empty((batch * segs, heads, dim), dtype=torch.float32, device=o.device)
-    decay = torch.empty((n, heads, dim), dtype=torch.float32, device=o.device) if dim in (64, 128) else None
-    _check(_lib.mixlib().exl3_mix_gla_segmented(*args, segs, seg_len, _p(seg_state), _p(seg_decay), _p(decay), code(q_view.dtype), _stream(o)))
+    tail = (code(q_view.dtype), _stream(o))
+    if dim in (64, 128) and rank <= 64:
+        decay = torch.empty((n, heads, dim), dtype=torch.float32, device=o.device)
+        _check(_lib.mixlib().exl3_mix_gla_chunked(*args, segs, seg_len, _p(seg_state), _p(seg_decay), _p(decay), *tail))
+    else:
+        _check(_lib.mixlib().exl3_mix_gla_segmented(*args, segs, seg_len, _p(seg_state), _p(seg_decay), *tail))
 
 
 def gla_out(out, o, w, g_view, eps: float):

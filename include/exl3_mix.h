@@ -48,7 +48,7 @@ extern "C" {
 #define EXL3_MIX_MASK_WINDOW 0
 #define EXL3_MIX_MASK_CHUNK  1
 
-#define EXL3_MIX_ABI_VERSION 6
+#define EXL3_MIX_ABI_VERSION 7     /* bumped whenever a symbol is added, removed or changes its arguments or meaning */
 
 const char* exl3_mix_last_error(void);
 int  exl3_mix_abi_version(void);
@@ -108,12 +108,16 @@ int exl3_mix_gla_scan(float* o, float* state, const void* q, int64_t q_ld, const
 /* The same results (up to float32 rounding) for long prompts, with the time axis cut into `segs` segments of `seg_len` rows per sequence
  * (segs * seg_len >= the longest sequence of the step) that run in parallel: every segment first runs from a zero state and leaves its local
  * state and the product of its decays, a short pass chains these into the state each segment starts from (and the slot's final state), and
- * every segment runs again from there and writes its outputs.  seg_state [batch*segs][heads][dim][vdim], seg_decay [batch*segs][heads][dim]: scratch.
- * decay (scratch [n][heads][dim], n the step's rows; may be null): with it, dim 64 or 128 and rank <= 64, the passes run in chunks of 16 rows on the matrix instructions. */
+ * every segment runs again from there and writes its outputs.  seg_state [batch*segs][heads][dim][vdim], seg_decay [batch*segs][heads][dim]: scratch. */
 int exl3_mix_gla_segmented(float* o, float* state, const void* q, int64_t q_ld, const void* k, int64_t k_ld, const void* v, int64_t v_ld,
                            const void* lr, int64_t lr_ld, const void* a2, const float* a2_bias, const int32_t* cu, const int32_t* slots, const int32_t* pos0,
                            int batch, int heads, int dim, int vdim, int rank, float tau, float q_scale, int segs, int seg_len,
-                           float* seg_state, float* seg_decay, float* decay, int dtype, void* stream);
+                           float* seg_state, float* seg_decay, int dtype, void* stream);
+/* exl3_mix_gla_segmented with its passes in chunks of 16 rows on the matrix instructions: dim 64 or 128, rank <= 64.  decay [n][heads][dim], n the step's rows: scratch. */
+int exl3_mix_gla_chunked(float* o, float* state, const void* q, int64_t q_ld, const void* k, int64_t k_ld, const void* v, int64_t v_ld,
+                         const void* lr, int64_t lr_ld, const void* a2, const float* a2_bias, const int32_t* cu, const int32_t* slots, const int32_t* pos0,
+                         int batch, int heads, int dim, int vdim, int rank, float tau, float q_scale, int segs, int seg_len,
+                         float* seg_state, float* seg_decay, float* decay, int dtype, void* stream);
 
 /* out[n][h*vdim + v] = o[n][h][v] / sqrt(mean_v(o[n][h]^2) + eps) * w[v] * silu(g[n][h*vdim + v]) */
 int exl3_mix_gla_out(void* out, const float* o, const float* w, const void* g, int64_t g_ld, float eps, int n, int heads, int vdim, int dtype, void* stream);
