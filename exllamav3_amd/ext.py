@@ -300,6 +300,15 @@ def dgemm(x: torch.Tensor, trellis: list, ys: list, suhs: list, svhs: list, mcg:
                         int(force_split), _raw_stream(x.get_device())))
 
 
+def _group_tile(rows: int, groups: int) -> int:
+    return -(-rows // groups) + max(4, rows // groups // 8)          # a group's expected rows, with room for an uneven routing
+
+
+def dgemm_grouped_fits(rows: int, groups: int, k: int) -> bool:
+    """Whether dgemm_grouped takes `rows` rows of k columns: the rotated rows of one matrix, padding included, stay below the 2 GiB that its 32-bit offsets reach."""
+    return _lib.lib().exl3_dgemm_grouped_xh_rows(rows, _group_tile(rows, groups)) * k * 2 <= 0x7fffffff
+
+
 def dgemm_grouped(x: torch.Tensor, row_map: torch.Tensor | None, group_rows: torch.Tensor, tables: tuple, ys: list, rows: int, K: int, mcg: bool, mul1: bool,
                   act_u: torch.Tensor | None = None) -> None:
     """exl3_dgemm over groups of rows (experts): output row r of ys[i] is x[row_map[r]] (r without a map; silu(x) * act_u with act_u) times matrix i of r's group.
@@ -312,7 +321,7 @@ def dgemm_grouped(x: torch.Tensor, row_map: torch.Tensor | None, group_rows: tor
     _req(row_map is not None or x.shape[0] >= rows, "dgemm_grouped: x has too few rows")
     _req(all(t.dtype == torch.long and t.is_contiguous() and t.numel() == cnt * groups for t in tables), "dgemm_grouped: pointer tables")
     _req(all(y.dim() == 2 and y.shape == (rows, n) and y.is_contiguous() and y.dtype == ys[0].dtype and y.dtype in (torch.half, torch.float) for y in ys), "dgemm_grouped: outputs")
-    tile = -(-rows // groups) + max(4, rows // groups // 8)          # a group's expected rows, with room for an uneven routing
+    tile = _group_tile(rows, groups)
     l = _lib.lib()
     need = l.exl3_dgemm_grouped_xh_rows(rows, tile)
     xh = torch.empty((cnt * need, k), dtype=torch.half, device=x.device)

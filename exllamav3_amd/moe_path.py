@@ -169,6 +169,11 @@ class SyntheticEXL3MoE:
         ext.exl3_mgemm_act_fx(slab, S, self.gu_svh, self.E, self.d_B, self.d_suh, self.d_svh, self.sel.view(-1), self.w.view(-1), R, self.K, mcg, mul1,
                               self.inter, m=1, num_tokens=1, force_split=sd)
 
+    def _on_packed_weights(self, rows: int) -> bool:
+        """Whether the grouped products of `rows` assignments decode the packed weights themselves: few enough rows per expert, and rotated rows (of the gate / up products and of
+        the down product) that ext.dgemm_grouped takes -- 256 experts of a hidden size of 7168 reach its 2 GiB at 18 700 tokens, below the row limit."""
+        return rows <= self.DGEMM_ROWS * self.E and all(ext.dgemm_grouped_fits(rows, self.E, k) for k in (self.hidden, self.inter))
+
     def forward_prefill(self, x: torch.Tensor) -> torch.Tensor:
         """The block for a prefill chunk (rows > the decode tiers): the large-batch tier of BlockSparseMLP.forward (modules/block_sparse_mlp.py:1169-1330).
         Every expert local: assignments grouped by expert on the device (ext.moe_group), two grouped products, a weighted sum per token -- no host synchronisation.  Otherwise:
@@ -196,7 +201,7 @@ class SyntheticEXL3MoE:
             g0, d0 = self.gate[0], self.down[0]
             token_sorted, pos, rows = ext.moe_group(sel, self.E)
             D = torch.empty((R, self.hidden), dtype=torch.float, device=dev)
-            if R <= self.DGEMM_ROWS * self.E and x.data_ptr() % 16 == 0 and x.stride(1) == 1:
+            if self._on_packed_weights(R) and x.data_ptr() % 16 == 0 and x.stride(1) == 1:
                 # a medium number of rows per expert: the packed weights decoded next to the products (ext.dgemm_grouped), no full-size weights in memory
                 gu = torch.empty((2, R, self.inter), dtype=torch.half, device=dev)
                 ext.dgemm_grouped(x, token_sorted, rows, (self.gu_B, self.gu_suh, self.gu_svh), [gu[0], gu[1]], R, g0.K, g0.mcg, g0.mul1)
