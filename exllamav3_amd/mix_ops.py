@@ -27,13 +27,16 @@ def _p(t):
     return None if t is None else t.data_ptr()
 
 
-def _stream(t: torch.Tensor):
-    return torch._C._cuda_getCurrentRawStream(t.get_device())
-
-
 def _req(cond, msg):
     if not cond:
         raise RuntimeError(msg)
+
+
+def _stream(t: torch.Tensor):
+    # (the raw handle of the current stream costs a twentieth of the Stream object; it takes device -1 of a host tensor for the current device, so that is refused here: a kernel must not get
+    # host addresses)
+    _req(t.is_cuda, "mix_ops: tensors must be on a GPU device")
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def _view(t: torch.Tensor, cols: int, name: str) -> int:
