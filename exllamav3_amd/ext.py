@@ -273,7 +273,7 @@ def dgemm(x: torch.Tensor, trellis: list, ys: list, suhs: list, svhs: list, mcg:
     _req(x.dim() == 2 and x.dtype == torch.half and x.stride(1) == 1, "dgemm: x must be 2-D float16 with a unit column stride")
     _req(1 <= K <= 8, "dgemm: packed must be 3-D int16, shared k and K")
     out = 2 if accumulate else int(ys[0].dtype == torch.float)
-    want, half, ns = (torch.float if out == 1 else torch.half), torch.half, []
+    want, half, ns, dev = (torch.float if out == 1 else torch.half), torch.half, [], x.get_device()
     for i in range(cnt):
         t, y, su, sv = trellis[i], ys[i], suhs[i], svhs[i]
         tk, tn, tw = t.shape
@@ -283,6 +283,7 @@ def dgemm(x: torch.Tensor, trellis: list, ys: list, suhs: list, svhs: list, mcg:
         _req(su.dtype == half and sv.dtype == half and su.numel() == k and sv.numel() == n and su.is_contiguous() and sv.is_contiguous(), "dgemm: suh / svh")
         b = biases[i] if biases else None
         _req(b is None or (b.dtype == half and b.numel() == n and b.is_contiguous()), "dgemm: bias")
+        _req(t.get_device() == y.get_device() == su.get_device() == sv.get_device() == dev and (b is None or b.get_device() == dev), "dgemm: every tensor must be on x's device")
         ns.append(n)
     if m == 0:
         return
@@ -297,7 +298,7 @@ def dgemm(x: torch.Tensor, trellis: list, ys: list, suhs: list, svhs: list, mcg:
     _check(l.exl3_dgemm(x.data_ptr(), x.stride(0), ptrs(*su), p + 4 * nf, rows.value, ptrs(*[t.data_ptr() for t in trellis]), ptrs(*[t.data_ptr() for t in svhs]),
                         ptrs(*[_p(b) for b in biases]) if biases else None, ptrs(*[t.data_ptr() for t in ys]),
                         (ctypes.c_int64 * cnt)(*[y.stride(0) for y in ys]), (ctypes.c_int * cnt)(*ns), cnt, out, p if nf else None, nf, m, k, K, _cb(mcg, mul1),
-                        int(force_split), _raw_stream(x.get_device())))
+                        int(force_split), _raw_stream(dev)))
 
 
 def _group_tile(rows: int, groups: int) -> int:
@@ -321,6 +322,7 @@ def dgemm_grouped(x: torch.Tensor, row_map: torch.Tensor | None, group_rows: tor
     _req(row_map is not None or x.shape[0] >= rows, "dgemm_grouped: x has too few rows")
     _req(all(t.dtype == torch.long and t.is_contiguous() and t.numel() == cnt * groups for t in tables), "dgemm_grouped: pointer tables")
     _req(all(y.dim() == 2 and y.shape == (rows, n) and y.is_contiguous() and y.dtype == ys[0].dtype and y.dtype in (torch.half, torch.float) for y in ys), "dgemm_grouped: outputs")
+    _req(all(t is None or t.get_device() == x.get_device() for t in (row_map, group_rows, act_u, *tables, *ys)), "dgemm_grouped: every tensor must be on x's device")
     tile = _group_tile(rows, groups)
     l = _lib.lib()
     need = l.exl3_dgemm_grouped_xh_rows(rows, tile)
@@ -541,6 +543,7 @@ def moe_combine(D: torch.Tensor, pos: torch.Tensor, weights: torch.Tensor) -> to
     _req(D.dtype == torch.float and D.dim() == 2 and D.is_contiguous() and D.shape[1] % 4 == 0, "moe_combine: D must be contiguous float32 (rows, hidden)")
     _req(pos.dtype == torch.int32 and weights.dtype == torch.half and pos.shape == weights.shape and pos.is_contiguous() and weights.is_contiguous() and 1 <= pos.shape[1] <= 64,
          "moe_combine: pos int32 and weights float16, (tokens, top_k), top_k at most 64")
+    _req(pos.get_device() == weights.get_device() == D.get_device(), "moe_combine: every tensor must be on D's device")
     out = torch.empty((pos.shape[0], D.shape[1]), dtype=torch.float, device=D.device)
     _check(_lib.lib().exl3_moe_combine(_p(D), _p(pos), _p(weights), _p(out), out.shape[0], pos.shape[1], D.shape[1], _stream(D)))
     return out

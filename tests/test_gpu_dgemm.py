@@ -150,3 +150,36 @@ def test_input_off_sixteen_bytes_keeps_its_route(rows):
     x = torch.randn((rows * k + 4,), device=_dev(), generator=torch.Generator(device=_dev()).manual_seed(rows)).half()[4:].view(rows, k)
     assert x.data_ptr() % 16 == 8 and x.is_contiguous()
     assert _err(lin.forward(x, {"no_reconstruct": True}), exact(x)) < 6e-4
+
+
+@pytest.mark.parametrize("host", ["trellis", "suh", "svh", "bias", "out"])
+def test_dgemm_refuses_tensors_of_another_device(host):
+    """A linear whose weights are still in host memory ended in an error on the fp16-weight route and does here: no host address reaches a kernel."""
+    from exllamav3_amd import ext
+    from exllamav3_amd.linear import LinearEXL3
+    (tr, su, sv), _ = _lin(256, 128, 4, 2, 5)
+    t = {"trellis": tr, "suh": su, "svh": sv, "bias": torch.zeros(128, dtype=torch.half, device=_dev())}
+    x = torch.zeros((200, 256), dtype=torch.half, device=_dev())
+    y = torch.zeros((200, 128), dtype=torch.half, device="cpu" if host == "out" else _dev())
+    if host != "out":
+        t[host] = t[host].cpu()
+        with pytest.raises(RuntimeError):
+            LinearEXL3(256, 128, t["trellis"], t["suh"], t["svh"], mul1=True, bias=t["bias"]).forward(x)
+    with pytest.raises(RuntimeError, match="device"):
+        ext.dgemm(x, [t["trellis"]], [y], [t["suh"]], [t["svh"]], False, True, [t["bias"]])
+
+
+def test_grouped_calls_refuse_tensors_of_another_device():
+    from exllamav3_amd import ext
+    dev = _dev()
+    bounds, tab = torch.tensor([0, 4], dtype=torch.int32, device=dev), tuple(torch.zeros(1, dtype=torch.long, device=dev) for _ in range(3))
+    x, y, pick = torch.zeros((4, 256), dtype=torch.half, device=dev), torch.zeros((4, 128), device=dev), torch.zeros(4, dtype=torch.long, device=dev)
+    for args in ((x, pick.cpu(), bounds, tab, [y]), (x, pick, bounds.cpu(), tab, [y]), (x, pick, bounds, tab[:2] + (tab[2].cpu(),), [y]), (x, pick, bounds, tab, [y.cpu()])):
+        with pytest.raises(RuntimeError, match="device"):
+            ext.dgemm_grouped(*args, 4, 4, False, True)
+    with pytest.raises(RuntimeError, match="device"):
+        ext.dgemm_grouped(x, None, bounds, tab, [y], 4, 4, False, True, act_u=x.cpu())
+    D, pos, w = torch.zeros((4, 128), device=dev), torch.zeros((2, 2), dtype=torch.int32, device=dev), torch.zeros((2, 2), dtype=torch.half, device=dev)
+    for args in ((D, pos.cpu(), w), (D, pos, w.cpu())):
+        with pytest.raises(RuntimeError, match="device"):
+            ext.moe_combine(*args)
