@@ -42,7 +42,8 @@ def _dgemm_ok(x: torch.Tensor, lins, rows: int) -> bool:
     most = DGEMM_MAX_ROWS_LONG_K if lins[0].in_features >= 2 * n else (DGEMM_MAX_ROWS_FEW_N if n <= DGEMM_FEW_N else DGEMM_MAX_ROWS)
     return (rows <= most and x.is_cuda and x.dtype == torch.half and x.data_ptr() % 16 == 0 and (x.dim() < 2 or x.stride(-2) % 8 == 0) and LinearEXL3.ahead is None
             and not LinearEXL3.cache_reconstructed and len({(l.K, l.mcg, l.mul1) for l in lins}) == 1
-            and all(l.in_features % 128 == 0 and l.out_features % 128 == 0 for l in lins))
+            and all(l.in_features % 128 == 0 and l.out_features % 128 == 0 and (l.bias is None or (l.bias.dtype == torch.half and l.bias.shape == (l.out_features,) and l.bias.is_contiguous()))
+                    for l in lins))
 
 
 def _dgemm(x: torch.Tensor, lins, ys, accumulate: bool = False) -> None:

@@ -183,3 +183,20 @@ def test_grouped_calls_refuse_tensors_of_another_device():
     for args in ((D, pos.cpu(), w), (D, pos, w.cpu())):
         with pytest.raises(RuntimeError, match="device"):
             ext.moe_combine(*args)
+
+
+@pytest.mark.parametrize("form", ["bfloat16", "strided", "one"])
+def test_a_bias_of_another_form_keeps_its_route(form):
+    """What `y += bias` takes and a kernel's pointer does not: other types, strides, one value for all columns."""
+    from exllamav3_amd.linear import LinearEXL3
+    k, n, K, rows = 256, 256, 4, 200
+    (tr, su, sv), exact = _lin(k, n, K, 2, 23)
+    gen = torch.Generator(device=_dev()).manual_seed(4)
+    bias = {"bfloat16": torch.randn(n, device=_dev(), generator=gen).bfloat16(), "strided": torch.randn(2 * n, device=_dev(), generator=gen).half()[::2],
+            "one": torch.randn(1, device=_dev(), generator=gen).half()}[form]
+    x = torch.randn((rows, k), device=_dev(), generator=gen).half()
+    y = LinearEXL3(k, n, tr, su, sv, mul1=True, bias=bias).forward(x)
+    assert _err(y, exact(x) + bias.double()) < 6e-4       # (x W and the sum rounded once each)
+    lin = LinearEXL3(k, n, tr, su, sv, mul1=True, bias=bias)
+    q, p = LinearEXL3.forward_separate([lin, LinearEXL3(k, n, tr, su, sv, mul1=True)], x)
+    assert torch.equal(q, y) and _err(p, exact(x)) < 6e-4
