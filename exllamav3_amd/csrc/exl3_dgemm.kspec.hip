@@ -81,8 +81,10 @@ void exl3_dgemm_kernel(const DgemmArgs a)
     const int mj = lane & 15, kg = lane >> 4;
     const int lds_r = mj * 256 + (((8 * kh + 2 * kg) ^ mj) << 4);
 
-    auto block = [&] (int b, int buf, LaneWords<K> (&slot)[2]) __attribute__((always_inline))
+    // (the last block of a slice with an odd number of them requests nothing: what lands in LDS behind its barrier would land in the output tile)
+    auto block = [&] (int b, int buf, LaneWords<K> (&slot)[2], auto last) __attribute__((always_inline))
     {
+        constexpr bool MORE = !decltype(last)::value;
         // the next block's activations are requested between the decode groups (every wave read that buffer for the last time in front of the barrier behind us):
         // back to back the requests of four waves queue at the CU's one address unit and hold their waves there
         half8_t bf[2][2][2];                              // [u][column c / c + 8][k half]
@@ -106,13 +108,16 @@ void exl3_dgemm_kernel(const DgemmArgs a)
                 union { half4_t h; uint32_t w[2]; } ux, uy; ux.h = x[0]; uy.h = y[0];
                 o[0][0].w[q] = ux.w[0]; o[0][1].w[q] = ux.w[1]; o[1][0].w[q] = uy.w[0]; o[1][1].w[q] = uy.w[1];
                 __builtin_amdgcn_sched_barrier(0);      // eight weights in flight: the registers are the accumulators' and the operands'
-                if (4 * u + q < MT) fetch(b + 1, buf ^ 1, 4 * u + q, 4 * u + q + 1);
+                if (MORE && 4 * u + q < MT) fetch(b + 1, buf ^ 1, 4 * u + q, 4 * u + q + 1);
             });
             bf[u][0][0] = o[0][0].h; bf[u][0][1] = o[0][1].h; bf[u][1][0] = o[1][0].h; bf[u][1][1] = o[1][1].h;
         }
-        asm volatile("" ::: "memory");                    // the words are requested behind the activations: the wait below counts them
-        #pragma unroll
-        for (int u = 0; u < 2; ++u) load_lane_words<K>(slot[u], wptr(b + NR, u));
+        if constexpr (MORE)
+        {
+            asm volatile("" ::: "memory");                // the words are requested behind the activations: the wait below counts them
+            #pragma unroll
+            for (int u = 0; u < 2; ++u) load_lane_words<K>(slot[u], wptr(b + NR, u));
+        }
         const char* ab = smem + buf * (BM * 256);
         #pragma unroll
         for (int i = 0; i < MT; ++i)
@@ -127,12 +132,12 @@ void exl3_dgemm_kernel(const DgemmArgs a)
                     acc[i][u][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af, bf[u][1][h], acc[i][u][1], 0, 0, 0);
                 }
             }
-        asm volatile("s_waitcnt vmcnt(%0)" :: "n"(WL) : "memory");
+        if constexpr (MORE) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(WL) : "memory");
         barrier();
     };
     int b = b0;
-    for (; b + 2 <= b1; b += 2) { block(b, 0, ring[0]); block(b + 1, 1, ring[NR - 1]); }
-    if (b < b1) block(b, 0, ring[0]);
+    for (; b + 2 <= b1; b += 2) { block(b, 0, ring[0], std::false_type{}); block(b + 1, 1, ring[NR - 1], std::false_type{}); }
+    if (b < b1) block(b, 0, ring[0], std::true_type{});
 
     dg_epilogue<MT>(a, t, acc, (float*) smem, wave, lane);
 }

@@ -120,14 +120,16 @@ void exl3_dgemm_wide_kernel(const DgemmArgs a)
     const int mj = lane & 15, kg = lane >> 4;
     const int lds_r = mj * 256 + (((8 * kh + 2 * kg) ^ mj) << 4);
 
-    auto block = [&] (int b, auto parity, LaneWords<K> (&slot)[2]) __attribute__((always_inline))
+    // (the last block of a slice with an odd number of them requests and decodes nothing: what lands in LDS behind its barrier would land in the output tile)
+    auto block = [&] (int b, auto parity, LaneWords<K> (&slot)[2], auto last) __attribute__((always_inline))
     {
         constexpr int buf = decltype(parity)::value;
+        constexpr bool MORE = !decltype(last)::value;
         const char* ab = smem + buf * (BM * 256);
         half8_t af[4];
         auto read = [&] (int gi) { af[gi & 3] = *((const half8_t*) (ab + (lds_r ^ ((gi & 1) << 4)) + (gi >> 1) * 4096)); };
         read(0); read(1); read(2);
-        words(slot);
+        if constexpr (MORE) words(slot);
         __builtin_amdgcn_sched_barrier(0);
         dg_static_for<0, G>([&] (auto gc)
         {
@@ -137,21 +139,24 @@ void exl3_dgemm_wide_kernel(const DgemmArgs a)
             {
                 constexpr int m = decltype(mc)::value, n = 4 * gi + m, u = m >> 1, set = m & 1;
                 dg_mfma(acc[i][u][set], af[gi & 3], bf[buf][u][set][h].h);
-                dg_static_for<n * 128 / NM, (n + 1) * 128 / NM>([&] (auto pc) { piece(pc, bf[buf ^ 1]); });
-                if constexpr (n % 3 == 1 && n / 3 < MT) fetch(b + 1, buf ^ 1, n / 3);
+                if constexpr (MORE) dg_static_for<n * 128 / NM, (n + 1) * 128 / NM>([&] (auto pc) { piece(pc, bf[buf ^ 1]); });
+                if constexpr (MORE && n % 3 == 1 && n / 3 < MT) fetch(b + 1, buf ^ 1, n / 3);
                 __builtin_amdgcn_sched_barrier(0);
             });
         });
-        #pragma unroll
-        for (int u = 0; u < 2; ++u) load_lane_words<K>(slot[u], wptr(b + 3, u));
-        asm volatile("s_waitcnt vmcnt(%0)" :: "n"(WL) : "memory");
+        if constexpr (MORE)
+        {
+            #pragma unroll
+            for (int u = 0; u < 2; ++u) load_lane_words<K>(slot[u], wptr(b + 3, u));
+            asm volatile("s_waitcnt vmcnt(%0)" :: "n"(WL) : "memory");
+        }
         barrier();
     };
     constexpr auto even = std::integral_constant<int, 0>{};
     constexpr auto odd = std::integral_constant<int, 1>{};
     int b = b0;
-    for (; b + 2 <= b1; b += 2) { block(b, even, ring[1]); block(b + 1, odd, ring[0]); }
-    if (b < b1) block(b, even, ring[1]);
+    for (; b + 2 <= b1; b += 2) { block(b, even, ring[1], std::false_type{}); block(b + 1, odd, ring[0], std::false_type{}); }
+    if (b < b1) block(b, even, ring[1], std::true_type{});
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");    // the last matrix instructions have written their accumulators
     __builtin_amdgcn_sched_barrier(0);
 
