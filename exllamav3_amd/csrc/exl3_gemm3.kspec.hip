@@ -1,4 +1,4 @@
-// EXL3 quantized small-m GEMM for gfx950, kernel generation 3 ("decode -> 16x16x32 MFMA straight from the decoding lane's registers"), 5..32 rows per pass.
+// EXL3 quantized small-m GEMM for gfx950, kernel generation 3 ("decode -> 16x16x32 MFMA straight from the decoding lane's registers"), 5..64 rows per pass.
 //
 //   C = ((A * suh) H) @ dequant(B) H * svh (+ bias)        reference: quant/exl3_gemm_kernel.cuh:8-80, quant/exl3_gemm_inner.cuh
 //                                                          (semantics only; the reference streams 16 rows per pass)
@@ -54,8 +54,9 @@ __device__ __forceinline__ void g3_static_for(F&& f)
 constexpr int g3_waves_per_eu(int K, int MT, bool ROT, bool RAW)
 {
     (void) RAW;                                      // the raw variant is instantiated for the rotated-input prologue only, whose budgets cover its row-sum accumulators
+    if (MT == 4 && K == 7 && !ROT) return 2;         // (round 4, likewise: 7-word ring slots)
     if (MT == 2 && K == 3 && !ROT) return 4;         // (round 4: the step-granular ring needs 2 more registers here than the 96 of five waves per SIMD)
-    return (K >= 7 || (ROT && K >= 5)) ? 3 : ((ROT || K >= 5) ? 4 : 5);
+    return MT == 4 ? (ROT ? (K >= 5 ? 2 : 3) : ((K == 4 || K <= 2) ? 4 : 3)) : ((K >= 7 || (ROT && K >= 5)) ? 3 : ((ROT || K >= 5) ? 4 : 5));
 }
 // waves per workgroup an instantiation can run with: 16 waves on 4 SIMDs need the 4-waves-per-SIMD register budget (128 VGPRs), 8 waves the 2-waves one
 constexpr bool g3_nwt_ok(int K, int MT, bool ROT, bool RAW, int NWT) { return NWT == 4 || (MT == 1 && g3_waves_per_eu(K, MT, ROT, RAW) >= NWT / 4); }
@@ -67,7 +68,7 @@ template <int K, int CB, int MT, bool ROT, bool RAWV, int NWT>
 // fp16-weight variant).  Removes a v_pk_fma_f16 per weight pair, 14 % of the streaming loop's VALU instructions; the same arithmetic as generation
 // 2's / 4's default variant.
 // ROT: the input is already rotated (fused decode pipeline) -- a separate instantiation so that neither prologue's registers burden the other.
-// five 4-wave workgroups per CU (LDS: 5 x 31 KB) need <= 96 VGPRs; the ROT prologue (16 registers of activation copy in
+// five 4-wave workgroups per CU (LDS: 5 x 31 KB) need <= 96 VGPRs; the 64-row passes, the ROT prologue (16 registers of activation copy in
 // flight next to the weight ring) and the wide rings of K >= 5 take the next register budgets instead of spilling (any scratch use slows
 // every launch); the table below is what hipcc 7.2 needs for zero scratch in every (K, codebook, MT, ROT) instantiation
 __global__ __launch_bounds__(64 * NWT) __attribute__((amdgpu_waves_per_eu(g3_waves_per_eu(K, MT, ROT, RAWV && CB == EXL3_CB_MUL1))))
@@ -148,7 +149,7 @@ void exl3_gemm3_kernel(const GemvArgs a)
     float4_t rsum[RAW ? MT : 1];
     #pragma unroll
     for (int i = 0; i < (RAW ? MT : 1); ++i) rsum[i] = float4_t{ 0.f, 0.f, 0.f, 0.f };
-    constexpr bool RSUM_EARLY = MT == 1;             // the 32-row passes fetch them in the epilogue instead (their register budgets are full)
+    constexpr bool RSUM_EARLY = MT == 1;             // the 32- / 64-row passes fetch them in the epilogue instead (their register budgets are full)
     if constexpr (RAW && RSUM_EARLY)
     {
         // the 16 lanes that share these rows (one DPP row) take different blocks each: one round of 4 loads per lane covers 16 blocks, nothing waits
@@ -179,7 +180,7 @@ void exl3_gemm3_kernel(const GemvArgs a)
     };
     // already rotated input (glue_rotate / glue_act): a straight copy in 16-byte pieces.  A row of the chunk is <= 2^cp_sl pieces; thread =
     // (row tid >> cp_sl of the instruction's 256 >> cp_sl rows, piece tid & (2^cp_sl - 1)); four instructions in flight per thread, so one batch
-    // covers 16 rows at up to 4 blocks per chunk (the decode shapes), 32 rows at 2
+    // covers 16 rows at up to 4 blocks per chunk (the decode shapes), 32 rows at 2, 64 rows at 1
     const int cp_sl = chb <= 1 ? 4 : (chb <= 2 ? 5 : (chb <= 4 ? 6 : (chb <= 8 ? 7 : (chb <= 16 ? 8 : 9))));       // (host: 16 chb <= 64 NWT)
     const int cp_piece = tid & ((1 << cp_sl) - 1), cp_rsub = tid >> cp_sl, cp_rows = (64 * NWT) >> cp_sl;
     auto copy_load = [&] (int c0, int cnt, int base, uint4_t (&v)[4])
@@ -243,7 +244,7 @@ void exl3_gemm3_kernel(const GemvArgs a)
         load_lane_words<K>(slot, step_ptr(refill));     // A/B: refill right after the words were copied out (the compiler then copies ring registers at the loop head and waits with vmcnt(0))
 #endif
 
-        // A operands of the step: 16-row passes request them before the decode and consume them after it (8 registers); the 32-row passes read
+        // A operands of the step: 16-row passes request them before the decode and consume them after it (8 registers); the 32- / 64-row passes read
         // them in front of each half's matrix instructions (their register budgets are full: any spill costs 1.5..3 us per launch)
         constexpr bool AF_EARLY = MT == 1;
         half8_t af[2][MT];
@@ -524,7 +525,8 @@ static void g3_launch_cb(int mt, bool raw, int nwt, dim3 grid, size_t lds, hipSt
     // the raw variant serves the fused decode pipeline (rotated input); the standalone op keeps the reference's fp16-rounded weights
     #define L(M, R) { if constexpr (CB == EXL3_CB_MUL1 && R) { if (raw) L2(M, R, true) else L2(M, R, false) } else L2(M, R, false) }
     if (mt == 1)      { if (rot) L(1, true) else L(1, false) }
-    else              { if (rot) L(2, true) else L(2, false) }
+    else if (mt == 2) { if (rot) L(2, true) else L(2, false) }
+    else              { if (rot) L(4, true) else L(4, false) }
     #undef L
     #undef L2
     #undef L3
@@ -533,7 +535,7 @@ static void g3_launch_cb(int mt, bool raw, int nwt, dim3 grid, size_t lds, hipSt
 #define G3_CAT_(a, b) a##b
 #define G3_CAT(a, b) G3_CAT_(a, b)
 
-// mt = row tiles of 16 per pass: 1 or 2; nwt = waves per workgroup: 4, 8 or 16 (exl3_gemm3_max_waves: what the instantiation can run with)
+// mt = row tiles of 16 per pass: 1, 2 or 4; nwt = waves per workgroup: 4, 8 or 16 (exl3_gemm3_max_waves: what the instantiation can run with)
 void G3_CAT(exl3_gemm3_launch_k, G2_K)(int cb, int mt, int var, int nwt, dim3 grid, size_t lds, hipStream_t st, const GemvArgs& args)
 {
     if (cb == 0) g3_launch_cb<0>(mt, false, nwt, grid, lds, st, args);

@@ -6,7 +6,7 @@
 // that is a whole number of 128-wide input Hadamard blocks, so BOTH rotations are workgroup-local: the input Hadamard is recomputed per
 // workgroup in the prologue from x (L2-resident) and the output Hadamard runs in the epilogue (S == 1), in the split-k reduce kernel below
 // (S > 1) or in the consumer of a deferred launch (exl3_glue.hip).  The kernels themselves: exl3_gemv2.kspec.hip (1..16 rows per weight
-// pass, column-pair-per-lane decode into v_mfma_f32_4x4x4_16B_f16) and exl3_gemm3.kspec.hip (5..32 rows, 16x16x32 MFMAs fed from the decoding lanes' registers).
+// pass, column-pair-per-lane decode into v_mfma_f32_4x4x4_16B_f16) and exl3_gemm3.kspec.hip (5..64 rows, 16x16x32 MFMAs fed from the decoding lanes' registers).
 // (The first-generation kernel of round 1 -- 4-wave workgroups, 16x16x32 MFMA on B-fragment-ordered lanes -- was an A/B baseline only and
 // has been removed; git history has it.)
 //
@@ -382,13 +382,14 @@ static int run_mgemm(const void* A, const void* const* Bs, void* const* Cs, cons
     if (!ctx) return EXL3_ERR_INIT;
 
     const int var = gemv_variant();
-    // generation 3 streams the weights once per up to 32 rows (exl3_gemm3.kspec.hip); the special input / output modes stay on generation 2
+    // generation 3 streams the weights once per up to 64 rows (exl3_gemm3.kspec.hip); the special input / output modes stay on generation 2
     const bool g3_ok = g_gemm3_min_rows > 0 && !in_norm && !tbl && !in_act && !epi && true;
-    // more than 32 rows: exl3_dgemm decodes every weight once per up to 256 rows where a pass of generation 3 would decode it once per 32 (4096 x 14336 at 64 / 100 / 128 rows:
+    // more than 32 rows: exl3_dgemm decodes every weight once per up to 256 rows where a pass of generation 3 decodes it once per 64 (4096 x 14336 at 64 / 100 / 128 rows:
     // 28 / 32 / 35 us, generation 3 in 64-row passes 30 / 58 / 59; at 32 rows and fewer generation 3 is ahead on small matrices, 14.6 against 17 us at 2048 x 2048)
     int dg_rows = m < 256 ? m : 256;
     if ((long) count * exl3_dgemm_xh_rows(dg_rows) * k * 2 > (long) EXL3_WS_XH_BYTES) dg_rows = m < 128 ? m : 128;
-    // (what exl3_dgemm does not take -- more than four matrices, buffers off its 16-byte pieces -- stays with the passes below)
+    // (what exl3_dgemm does not take -- buffers off its 16-byte pieces, rotated rows beyond the scratch -- stays with the passes below, 64 rows each: an input off 16 bytes takes
+    // 20.1 us at 64 x 4096 -> 4096 and 39.0 at 128, 32.5 and 64.0 in passes of 32; on 16 bytes exl3_dgemm takes 18.0 and 21.1)
     bool dg_ok = count <= 4 && (uintptr_t) A % 16 == 0;
     for (int i = 0; dg_ok && !tbl && Cs && i < count; ++i) dg_ok = (uintptr_t) Cs[i] % (c_fp32 ? 16 : 8) == 0;
     if (g3_ok && dg_ok && cpw == 0 && !deferred && !rotated && m > 32 && (long) count * exl3_dgemm_xh_rows(dg_rows) * k * 2 <= (long) EXL3_WS_XH_BYTES)
@@ -409,7 +410,7 @@ static int run_mgemm(const void* A, const void* const* Bs, void* const* Cs, cons
         }
         return 1;
     }
-    const int pass_rows = (g3_ok && !deferred && !rotated && m > 16) ? 32 : 16;
+    const int pass_rows = (g3_ok && !deferred && !rotated && m > 16) ? (m > 32 ? 64 : 32) : 16;
     for (int m0 = 0; m0 < m; m0 += pass_rows)
     {
         const int mp = (m - m0) < pass_rows ? (m - m0) : pass_rows;
@@ -439,11 +440,11 @@ static int run_mgemm(const void* A, const void* const* Bs, void* const* Cs, cons
             }
             pass_flags |= GEMV_IN_ROTATED;
         }
-        // generation 3: column blocks per workgroup and the split are chosen together (16-row passes; 32-row passes keep 4-wave workgroups)
+        // generation 3: column blocks per workgroup and the split are chosen together (16-row passes; 32- / 64-row passes keep 4-wave workgroups)
         int g3cpw = 1, g3fs = 0;
         if (g3)
         {
-            const int mt_ = mp > 16 ? 2 : 1;
+            const int mt_ = mp > 32 ? 4 : (mp > 16 ? 2 : 1);
             const int maxw = gemm3_max_waves(K, mt_, (pass_flags & GEMV_IN_ROTATED) ? 1 : 0);
             const int nbk = k / 128, cus = ctx->num_cus;
             int forced_S = 0;
@@ -587,7 +588,7 @@ static int run_mgemm(const void* A, const void* const* Bs, void* const* Cs, cons
         EXL3_CHECK_ARG(!(fxz.ptr && gen == 3), "exl3_fx_zero_next: the launch that followed cannot clear the buffer (not a generation-4 launch: rows > 4, a slice of more than 32 Hadamard blocks, a tail / wave-per-column-block mode, or generation 4 switched off)");
         if (gen == 3)
         {
-            const int mt = mp > 16 ? 2 : 1;
+            const int mt = mp > 32 ? 4 : (mp > 16 ? 2 : 1);
             // workgroup = 4 g3cpw waves = g3cpw adjacent column blocks of one matrix sharing ONE activation tile in LDS (16 rows keep a whole 8-block
             // slice resident at 4 waves, a whole k = 4096 at 16: one chunk, no second prologue / barrier inside the stream)
             const int nwt = 4 * g3cpw;

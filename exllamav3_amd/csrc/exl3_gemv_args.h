@@ -232,7 +232,7 @@ size_t exl3_gemv2_lds_bytes(int ng, int var, int cb, int nwv, int m, int chunk_b
 #define G2_DECL(KK) void exl3_gemv2_launch_k##KK(int cb, int var, int ng, int nwv, dim3 grid, size_t lds, hipStream_t st, const GemvArgs& args);
 G2_DECL(1) G2_DECL(2) G2_DECL(3) G2_DECL(4) G2_DECL(5) G2_DECL(6) G2_DECL(7) G2_DECL(8)
 #undef G2_DECL
-// generation 3 (exl3_gemm3.kspec.hip): 5..32 rows per pass through an LDS transpose into 16x16x32 MFMAs
+// generation 3 (exl3_gemm3.kspec.hip): 5..64 rows per pass through an LDS transpose into 16x16x32 MFMAs
 #define G3_DECL(KK) void exl3_gemm3_launch_k##KK(int cb, int mt, int var, int nwt, dim3 grid, size_t lds, hipStream_t st, const GemvArgs& args); \
                     int exl3_gemm3_max_waves_k##KK(int mt, int rot);
 G3_DECL(1) G3_DECL(2) G3_DECL(3) G3_DECL(4) G3_DECL(5) G3_DECL(6) G3_DECL(7) G3_DECL(8)

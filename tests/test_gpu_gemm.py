@@ -376,3 +376,43 @@ def test_gemm3_lm_head_width_at_64_rows_and_oversized_forced_split(dev):
     assert np.abs(g - ref).max() / np.sqrt((ref ** 2).mean()) < TOL
     # forced split beyond 64 slices (96 Hadamard blocks): normalised, not a crash
     assert _run(dev, 96 * 128, 256, 4, 2, 8, 1, force_split=80) < TOL
+
+
+@pytest.mark.parametrize("off", ["input", "output"])
+@pytest.mark.parametrize("rows", [64, 65, 128, 144])
+def test_buffers_off_sixteen_bytes_run_in_passes_of_64_rows(off, rows):
+    """What the medium-row kernels do not take streams the weights once per 64 rows: the launches of a recorded call are those of one pass times the passes, and the values those of the aligned call
+    to the roundings of the small-m kernels (fp16 input, intermediate and output: 6e-4)."""
+    import ctypes
+    from exllamav3_amd import ext
+    dev, k, n, K = torch.device("cuda:0"), 512, 512, 4
+    ext.init(0)
+    gen = torch.Generator(device=dev).manual_seed(rows)
+    tr = torch.randint(-32768, 32768, (k // 16, n // 16, 16 * K), dtype=torch.int16, device=dev, generator=gen)
+    su = (torch.randint(0, 2, (k,), device=dev, generator=gen) * 2 - 1).half()
+    sv = (torch.rand(n, device=dev, generator=gen) * 0.1).half()
+    x = torch.randn((rows * k + 4,), device=dev, generator=gen).half()
+
+    def call(rows_, shift_in, shift_out):
+        a = x[:rows_ * k].view(rows_, k)
+        if shift_in:
+            a = torch.cat([torch.zeros(4, dtype=torch.half, device=dev), a.reshape(-1)])[4:].view(rows_, k)
+        y = torch.zeros((rows_ * n + 2,), device=dev)[2 if shift_out else 0:][:rows_ * n].view(rows_, n)
+        run = lambda: ext.exl3_gemm(a, tr, y, su, None, sv, -1, False, True)
+        run()
+        graph, side = torch.cuda.CUDAGraph(keep_graph=True), torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.graph(graph, stream=side):
+            run()
+        count = ctypes.c_size_t(0)
+        hip = ctypes.CDLL(None)                               # (torch's own runtime, loaded with global symbols)
+        assert hip.hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(count)) == 0
+        torch.cuda.synchronize()
+        return y, count.value
+    y, nodes = call(rows, off == "input", off == "output")
+    _, one = call(64, off == "input", off == "output")
+    _, rest = call(rows % 64, off == "input", off == "output") if rows % 64 else (None, 0)
+    _, single = call(32, off == "input", off == "output")
+    want, _ = call(rows, False, False)
+    assert one == single and nodes == rows // 64 * one + rest
+    assert (y - want).norm() / want.norm() < 6e-4
