@@ -103,6 +103,8 @@ def _declare(l):
     sig("exl3_reconstruct", vp, vp, i32, i32, i32, i32, i64, i64, vp)
     sig("exl3_reconstruct_had", vp, vp, vp, vp, i32, i32, i32, i32, i64, i64, vp)
     sig("exl3_dgemm_plan", i32, i32, i32, ctypes.POINTER(i32), ctypes.POINTER(i64))
+    sig("exl3_dgemm_pays", i32, i32, i32, i32, i32)
+    sig("exl3_dgemm_plan_kind", i32, i32, i32, i32, i32, ctypes.POINTER(i32), ctypes.POINTER(i64))
     sig("exl3_dgemm", vp, i64, vp, vp, i32, vp, vp, vp, vp, vp, vp, i32, i32, vp, i64, i32, i32, i32, i32, i32, vp)
     sig("exl3_dgemm_grouped_xh_rows", i32, i32)
     sig("exl3_dgemm_grouped", vp, vp, i64, vp, vp, vp, i32, vp, vp, vp, i32, vp, i64, i32, i32, i32, i32, i32, i32, i32, i32, vp)

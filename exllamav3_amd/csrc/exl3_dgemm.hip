@@ -116,40 +116,50 @@ static int dg_row_tiles(int m)
     return m <= 128 ? dg_narrow_tiles(m, 1) : dg_wide_tiles(m, (m + 255) / 256);
 }
 
-struct DgPlan { int mt, mtiles, S; };
+struct DgPlan { int mt, mtiles, S; double us; };
 
-// Microseconds of one (m, k, n) product cut into `mtiles` row tiles and s k-slices of b blocks on `cus` compute units.
-// Up to 128 rows (one row tile), fitted to 4096 x 14336, 14336 x 4096, 4096 x 6144, 2048 x 2048: a workgroup pays its prologue and epilogue once and `step` per 128 k; alone on its CU
-// no less than 0.8 us, the latency of its own chain.
-// Above, fitted to those, 2048 x 8192 and 4096 x 4096 at 300 .. 1500 rows, both kernels, every row-tile count and split (about 900 launches, 3.6 % rms; its choices are 0.5 % slower than
-// the best ones on average, 10 % at most): a wide workgroup has its CU alone, a last round that fills the chip in part runs a little faster than a full one; two narrow workgroups
-// share a CU at about the cost of one after the other.
-// A split writes and reads its partial sums.
-static double dg_cost(int m, int k, int n, int mt, int mtiles, int s, int b, int cus)
+// What a block of 128 k costs beside 1 .. 4 bits of the hashed-byte codebook (cb 2): wider words are two loads per lane from 5 bits and unaligned ones at 7, the codebooks that add two halves
+// decode with more instructions.  wide: in the wide kernel, one / two: in the narrow one with one / two workgroups on a compute unit, deep: 7 and 8 bits in the narrow kernel's 112- and 128-row
+// forms, whose second ring of words does not fit the registers.
+struct DgKind { double wide, one, two, small, deep; };
+static DgKind dg_kind(int K, int cb)
+{
+    const int w5 = K > 4, w7 = K > 6, c1 = cb == 1, c0 = cb == 0;
+    return { 0.086 * w5 + 0.063 * w7 + 0.049 * c1 + 0.134 * c0, 0.103 * w5 + 0.054 * w7 + 0.172 * c1 + 0.223 * c0, 0.107 * w5 + 0.053 * w7 + 0.082 * c1 + 0.221 * c0,
+             0.076 * w5 + 0.038 * w7 + 0.068 * c1 + 0.134 * c0, (double) w7 };
+}
+
+// Microseconds of one (m, k, n) product cut into `mtiles` row tiles and s k-slices of b blocks on `cus` compute units, without the rotation in front of it.
+// Fitted to 38 800 launches: fourteen shapes from 2048 x 512 to 4096 x 14336, 40 .. 1000 rows, 2, 4, 6, 8 bits, three codebooks, every row tiling, up to five splits each.  The choices are 0.3 %
+// slower than the best of the launches on average up to 128 rows (7 % at most) and 0.9 % above (13 %); without the terms of dg_kind they were 1.0 % (30 %) and 5.2 % (48 %) slower:
+// 8192 x 8192, 8 bits, 420 rows 134 us, 84 now.
+// Up to 128 rows (one row tile): a workgroup pays its prologue and epilogue once and `step` per 128 k.  Above: a wide workgroup has its CU alone, a last round that fills the chip in part runs
+// faster than a full one; two narrow workgroups share a CU at about the cost of one after the other.  A split writes and reads its partial sums and launches their reduction.
+static double dg_cost(const DgKind& kind, int m, int k, int n, int mt, int mtiles, int s, int b, int cus)
 {
     const double wgs = (double) mtiles * (n >> 7) * s;
-    const double sums = s > 1 ? 1e-6 * s * (double) m * n : 0.0;
+    const double sums = s > 1 ? 1e-6 * s * (double) m * n : 0.0, deep = mt > 6 ? kind.deep : 0.0;
     if (m <= 128)
     {
-        const double per_cu = ceil(wgs / cus), step = per_cu == 1.0 ? 0.70 + 0.042 * mt : 0.30 + 0.10 * mt;
-        return per_cu * (b * step + (per_cu == 1.0 ? 8.0 : 5.0)) + (s > 1 ? 2.0 + sums : 0.0);
+        const double per_cu = ceil(wgs / cus), alone = 0.471 + 0.079 * mt + kind.small + 0.473 * deep, shared = 0.299 + 0.038 * mt + 0.83 * kind.small + 0.082 * deep;
+        return per_cu * (per_cu == 1.0 ? b * alone + 6.7 : b * shared + 6.1) + (s > 1 ? 1.6 + 1.45 * sums + 0.08 * s : 0.0);
     }
-    const double split = s > 1 ? 3.0 + 0.65 * sums : 0.0;
     if (mt > 8)
     {
         const double rounds = ceil(wgs / cus), last = wgs / cus - (rounds - 1.0);
-        return (rounds - 1.0 + 0.67 + 0.33 * last) * (b * (0.34 + 0.091 * mt) + 0.59 * mt) + split;
+        return (rounds - 1.0 + 0.86 + 0.14 * last) * (b * (0.156 + kind.wide + 0.081 * mt) + 0.69 * mt) + (s > 1 ? 2.2 + 0.27 * sums + 0.10 * s : 0.0);
     }
-    const double one = b * fmax(0.148 * mt, 0.70 + 0.042 * mt) + 0.9, two = b * (0.25 + 0.222 * mt) + 0.62 * mt;
+    const double one = b * (0.215 + kind.one + 0.112 * mt + 0.487 * deep) + 0.03 * mt, two = b * (0.828 + kind.two + 0.122 * mt) + 0.73 * mt;
     const double rounds = ceil(wgs / (2.0 * cus)), left = wgs - (rounds - 1.0) * 2.0 * cus;
-    return (rounds - 1.0) * two + (left > cus ? two * (0.73 + 0.27 * left / (2.0 * cus)) : one) + split;
+    return (rounds - 1.0) * two + (left > cus ? two * (0.50 + 0.50 * left / (2.0 * cus)) : one) + (s > 1 ? 3.4 + 0.36 * sums + 0.35 * s : 0.0);
 }
 
 // The cheapest kernel, row tiling and split whose partial sums fit max_floats
-static DgPlan dg_plan(int m, int k, int n, int cus, int64_t max_floats)
+static DgPlan dg_plan(int m, int k, int n, int K, int cb, int cus, int64_t max_floats)
 {
     const int nb = k >> 7;
-    DgPlan best = { 0, 0, 1 };
+    const DgKind kind = dg_kind(K, cb);
+    DgPlan best = { 0, 0, 1, 0.0 };
     double cost = 1e30;
     auto tiling = [&] (int mt, int mtiles, bool alone)
     {
@@ -159,8 +169,8 @@ static DgPlan dg_plan(int m, int k, int n, int cus, int64_t max_floats)
             if ((nb + b - 1) / b != s) continue;
             if (s > 1 && (int64_t) s * m * n > max_floats) break;
             if (alone && (int64_t) mtiles * (n >> 7) * s > cus) break;
-            const double c = dg_cost(m, k, n, mt, mtiles, s, b, cus);
-            if (c < cost) { cost = c; best = { mt, mtiles, s }; }
+            const double c = dg_cost(kind, m, k, n, mt, mtiles, s, b, cus);
+            if (c < cost) { cost = c; best = { mt, mtiles, s, c }; }
         }
     };
     if (m <= 128) tiling(dg_narrow_tiles(m, 1), 1, false);
@@ -211,16 +221,35 @@ int exl3_dgemm_xh_rows(int m)
     return rows;
 }
 
-extern "C" int exl3_dgemm_plan(int m, int k, int n, int* xh_rows, int64_t* slab_floats)
+extern "C" int exl3_dgemm_plan_kind(int m, int k, int n, int K, int cb, int* xh_rows, int64_t* slab_floats)
 {
     EXL3_CHECK_ARG(xh_rows && slab_floats && m >= 1 && k > 0 && n > 0 && k % 128 == 0 && n % 128 == 0, "exl3_dgemm_plan: m >= 1, k and n divisible by 128");
+    EXL3_CHECK_ARG(K >= 1 && K <= 8 && cb >= 0 && cb <= 2, "exl3_dgemm_plan: K must be in [1, 8], codebook in [0, 2]");
     int cus = 0;
     const int rc = dg_device_cus(&cus);
     if (rc != EXL3_OK) return rc;
-    const int S = dg_plan(m, k, n, cus, INT64_MAX).S;
+    const int S = dg_plan(m, k, n, K, cb, cus, INT64_MAX).S;
     *xh_rows = exl3_dgemm_xh_rows(m);
     *slab_floats = S > 1 ? (int64_t) S * m * n : 0;
     return EXL3_OK;
+}
+
+extern "C" int exl3_dgemm_plan(int m, int k, int n, int* xh_rows, int64_t* slab_floats) { return exl3_dgemm_plan_kind(m, k, n, 4, 2, xh_rows, slab_floats); }
+
+// Whether the product is faster here than through a rebuilt fp16 matrix and a plain GEMM (128 < m < 1024; both called one after the other, launches included).  Here: the rotation and the launches,
+// then the plan.  There: two launches; W^T written once, and for every 256 rows read again next to their products (its tiles), with a term for long contractions, whose few outputs leave compute
+// units idle.  Fitted to 3 510 calls (thirteen shapes, 150 .. 1000 rows, 1 .. 8 bits, three codebooks; 4.1 % and 3.6 % rms); the margin leaves 27 of them more than 2 % slower than the other route, 8 %
+// at most, and the mean 0.2 % above the better route's.  Row limits without a term for bits and codebook left 181 of them slower, 21 % at most (4096 x 6144, 8 bits, 560 rows: 69 us / 57).
+extern "C" int exl3_dgemm_pays(int m, int k, int n, int K, int cb)
+{
+    EXL3_CHECK_ARG(m >= 1 && k > 0 && n > 0 && k % 128 == 0 && n % 128 == 0 && K >= 1 && K <= 8 && cb >= 0 && cb <= 2, "exl3_dgemm_pays: m >= 1, k and n divisible by 128, K in [1, 8], codebook in [0, 2]");
+    int cus = 0;
+    const int rc = dg_device_cus(&cus);
+    if (rc != EXL3_OK) return rc;
+    const double kn = 1e-6 * (double) k * n, tiles = (m + 255) / 256;
+    const double here = fmax(16.5, 9.5 + 1.243 * dg_plan(m, k, n, K, cb, cus, INT64_MAX).us);
+    const double there = fmax(30.5, 15.3 + 0.669 * kn + 0.126 * kn * tiles + 0.616e-3 * kn * m + 0.88e-3 * k + 1.365e-6 * (double) k * m);
+    return here < 0.97 * there ? 1 : 0;
 }
 
 extern "C" int exl3_dgemm(const void* x, int64_t ldx, const void* const* suhs, void* xh, int xh_rows, const void* const* Bs, const void* const* svhs,
@@ -255,7 +284,7 @@ extern "C" int exl3_dgemm(const void* x, int64_t ldx, const void* const* suhs, v
         a.nblk += ns[i] / 128;
     }
     a.num_mats = count; a.m = m; a.k = k; a.out = out; a.xh_bytes = rows * k * 2;
-    DgPlan plan = dg_plan(m, k, 128 * a.nblk, cus, slab ? slab_floats : 0);
+    DgPlan plan = dg_plan(m, k, 128 * a.nblk, K, cb, cus, slab ? slab_floats : 0);
     if (force_split < 0 && m > 128) { plan.mtiles = (m + 255) / 256; plan.mt = dg_wide_tiles(m, plan.mtiles); }
     const int mt = plan.mt;
     a.mtiles = plan.mtiles;

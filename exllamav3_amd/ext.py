@@ -10,6 +10,7 @@ INTEGRATION.md shows how this module is installed under the name `exllamav3_ext`
 """
 from __future__ import annotations
 import ctypes
+import functools
 import torch
 from . import _lib
 from ._lib import check as _check
@@ -262,6 +263,23 @@ def exl3_gemm(A: torch.Tensor, B: torch.Tensor, C: torch.Tensor, suh: torch.Tens
                                        int(C.dtype == torch.float), int(force_split), _stream(A)))
 
 
+# (both are functions of sizes and the device alone)
+@functools.lru_cache(maxsize=4096)
+def dgemm_pays(device: int, m: int, k: int, n: int, K: int, mcg: bool, mul1: bool) -> bool:
+    """Whether dgemm takes less time for m rows of k and n output columns in all than a rebuilt fp16 matrix and a plain GEMM."""
+    with torch.cuda.device(device):
+        return _check(_lib.lib().exl3_dgemm_pays(m, k, n, K, _cb(mcg, mul1))) == 1
+
+
+@functools.lru_cache(maxsize=4096)
+def _dgemm_plan(device: int, m: int, k: int, n: int, K: int, cb: int) -> tuple[int, int]:
+    """(rows of the rotated-row buffer, floats of the partial sums) of a dgemm call."""
+    rows, floats = ctypes.c_int(0), ctypes.c_int64(0)
+    with torch.cuda.device(device):
+        _check(_lib.lib().exl3_dgemm_plan_kind(m, k, n, K, cb, ctypes.byref(rows), ctypes.byref(floats)))
+    return rows.value, floats.value
+
+
 def dgemm(x: torch.Tensor, trellis: list, ys: list, suhs: list, svhs: list, mcg: bool, mul1: bool, biases: list | None = None, accumulate: bool = False,
           force_split: int = 0) -> None:
     """ys[i] (=, or += with accumulate) x @ W_i (+ bias_i) for a medium number of rows (exl3_dgemm) and up to 4 matrices of one k, K and codebook: x is rotated once
@@ -288,16 +306,17 @@ def dgemm(x: torch.Tensor, trellis: list, ys: list, suhs: list, svhs: list, mcg:
     if m == 0:
         return
     l, ntot, ptrs = _lib.lib(), sum(ns), _vp * cnt
-    rows, floats = ctypes.c_int(0), ctypes.c_int64(0)
-    _check(l.exl3_dgemm_plan(m, k, ntot, ctypes.byref(rows), ctypes.byref(floats)))
-    nf = floats.value if force_split == 0 else abs(force_split) * m * ntot
+    cb = _cb(mcg, mul1)
+    rows, nf = _dgemm_plan(dev, m, k, ntot, K, cb)
+    if force_split:
+        nf = abs(force_split) * m * ntot
     su = [t.data_ptr() for t in suhs]
     distinct = cnt if cnt == 1 else len(set(su))
-    buf = torch.empty((2 * nf + distinct * rows.value * k,), dtype=half, device=x.device)        # partial sums (float32), then the rotated rows
+    buf = torch.empty((2 * nf + distinct * rows * k,), dtype=half, device=x.device)        # partial sums (float32), then the rotated rows
     p = buf.data_ptr()
-    _check(l.exl3_dgemm(x.data_ptr(), x.stride(0), ptrs(*su), p + 4 * nf, rows.value, ptrs(*[t.data_ptr() for t in trellis]), ptrs(*[t.data_ptr() for t in svhs]),
+    _check(l.exl3_dgemm(x.data_ptr(), x.stride(0), ptrs(*su), p + 4 * nf, rows, ptrs(*[t.data_ptr() for t in trellis]), ptrs(*[t.data_ptr() for t in svhs]),
                         ptrs(*[_p(b) for b in biases]) if biases else None, ptrs(*[t.data_ptr() for t in ys]),
-                        (ctypes.c_int64 * cnt)(*[y.stride(0) for y in ys]), (ctypes.c_int * cnt)(*ns), cnt, out, p if nf else None, nf, m, k, K, _cb(mcg, mul1),
+                        (ctypes.c_int64 * cnt)(*[y.stride(0) for y in ys]), (ctypes.c_int * cnt)(*ns), cnt, out, p if nf else None, nf, m, k, K, cb,
                         int(force_split), _raw_stream(dev)))
 
 

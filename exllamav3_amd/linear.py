@@ -5,7 +5,7 @@ of the C-ABI ops in exllamav3_amd.ext.
 
   forward(x, params, out_dtype):
      rows <= AUTO_RECONSTRUCT_THRESHOLD (144)  -> fused HIP GEMV / small-m GEMM (exl3.py:133-137)
-     rows <= DGEMM_MAX_ROWS (more for a long contraction) -> ext.dgemm: the packed weights decoded in registers once per row tile, no fp16 weight matrix
+     rows <= DGEMM_MAX_ROWS and sizes, bits and codebook for which it is faster (ext.dgemm_pays) -> ext.dgemm: packed weights decoded in registers once per row tile, no fp16 weight matrix
      otherwise reconstruct_hgemm (exl3.py:161-218):
         rows <  FUSED_RECONSTRUCT_MIN_ROWS: had_r_128(x, suh) -> reconstruct -> hgemm -> had_r_128(y, svh)
         rows >= FUSED_RECONSTRUCT_MIN_ROWS: reconstruct_had_slice (original-basis W, both Hadamards on the matrix pipe) -> hgemm on raw x
@@ -24,11 +24,9 @@ MAX_RECONSTRUCT_SLICE_N = 32768           # exl3.py:11
 FUSED_RECONSTRUCT_MIN_ROWS = AUTO_RECONSTRUCT_THRESHOLD + 1
 
 
-# Row counts that ext.dgemm takes.  Decoding a weight once per row tile costs more than writing and reading it as fp16 from some row count on; the plain GEMM leaves compute units idle for
-# longer where the outputs are few, most of all behind a long contraction.  Measured (us, dgemm / reconstruct + GEMM): 4096 x 14336 at 512 / 600 / 768 rows 76 / 85, 101 / 100, 116 / 111;
-# 2048 x 8192 at 600 / 768 / 900 rows 37 / 43, 42 / 44, 51 / 48; 4096 x 6144 at 768 / 1024 rows 58 / 63, 71 / 65; 14336 x 4096 at 768 / 1024 / 1500 rows 103 / 138, 130 / 158, 186 / 187.
-# The last limit stays below 1024, where prompt chunks may have their weights rebuilt ahead on a second stream (ReconstructAhead) and give the same bits either way.
-DGEMM_MAX_ROWS, DGEMM_MAX_ROWS_FEW_N, DGEMM_MAX_ROWS_LONG_K, DGEMM_FEW_N = 512, 768, 1023, 8192
+# ext.dgemm ends below this many rows: from 1024 on prompt chunks may have their weights rebuilt ahead on a second stream (ReconstructAhead) and give the same bits either way.  Below, sizes, bits per
+# weight and codebook decide (ext.dgemm_pays): 14336 x 4096 at 1000 rows 131 us against 148 through rebuilt weights (4 bits), 4096 x 14336 at 512 rows 77 / 83, at 560 rows 94 / 88.
+DGEMM_MAX_ROWS = 1023
 
 #: the fused prefill GEMMs reconstruct their matrices with ONE launch (ext.reconstruct_had_multi_t); EXL3_HIP_RECON_MULTI=0: one launch per matrix
 RECON_MULTI = os.environ.get("EXL3_HIP_RECON_MULTI", "1") != "0"
@@ -36,14 +34,17 @@ RECON_MULTI = os.environ.get("EXL3_HIP_RECON_MULTI", "1") != "0"
 
 def _dgemm_ok(x: torch.Tensor, lins, rows: int) -> bool:
     """Whether ext.dgemm takes (and should take) these linears of one input for `rows` rows."""
-    if rows > DGEMM_MAX_ROWS_LONG_K:
+    if not (rows <= DGEMM_MAX_ROWS and x.is_cuda and x.dtype == torch.half and x.data_ptr() % 16 == 0 and (x.dim() < 2 or x.stride(-2) % 8 == 0) and LinearEXL3.ahead is None
+            and not LinearEXL3.cache_reconstructed):
         return False
-    n = sum(l.out_features for l in lins)
-    most = DGEMM_MAX_ROWS_LONG_K if lins[0].in_features >= 2 * n else (DGEMM_MAX_ROWS_FEW_N if n <= DGEMM_FEW_N else DGEMM_MAX_ROWS)
-    return (rows <= most and x.is_cuda and x.dtype == torch.half and x.data_ptr() % 16 == 0 and (x.dim() < 2 or x.stride(-2) % 8 == 0) and LinearEXL3.ahead is None
-            and not LinearEXL3.cache_reconstructed and len({(l.K, l.mcg, l.mul1) for l in lins}) == 1
-            and all(l.in_features % 128 == 0 and l.out_features % 128 == 0 and (l.bias is None or (l.bias.dtype == torch.half and l.bias.shape == (l.out_features,) and l.bias.is_contiguous()))
-                    for l in lins))
+    l0, n = lins[0], 0
+    for l in lins:
+        b = l.bias
+        if (l.in_features % 128 or l.out_features % 128 or (l.K, l.mcg, l.mul1) != (l0.K, l0.mcg, l0.mul1)
+                or (b is not None and not (b.dtype == torch.half and b.shape == (l.out_features,) and b.is_contiguous()))):
+            return False
+        n += l.out_features
+    return ext.dgemm_pays(x.get_device(), rows, l0.in_features, n, l0.K, l0.mcg, l0.mul1)
 
 
 def _dgemm(x: torch.Tensor, lins, ys, accumulate: bool = False) -> None:

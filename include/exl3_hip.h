@@ -98,9 +98,11 @@ int exl3_had_r_128(const void* in, void* out, const void* pre_scale, const void*
  * registers once per row tile.  x: m rows of k fp16, row stride ldx.  out: 0 = fp16, 1 = fp32, 2 = C (fp16) += result, each
  * rounded once; 3 / 4 = fp16 / fp32 with the intermediate fp16 roundings of exl3_gemm's small-m kernels; ldcs: row strides of the outputs in elements.
  * xh: scratch for the rotated rows, xh_rows x k fp16 per distinct suh (rows >= m are read and may hold anything); slab: fp32 scratch for split sums or NULL.
- * exl3_dgemm_plan: the xh_rows and slab_floats that an (m, k, sum of n_i) product wants (less slab: fewer slices).  force_split != 0 sets the number of k-slices
- * (negative, m > 128: that many, in the 256-row kernel with the fewest row tiles). */
+ * exl3_dgemm_plan_kind: the xh_rows and slab_floats that an (m, k, sum of n_i) product of K bits and codebook cb wants (less slab: fewer slices); exl3_dgemm_plan: at 4 bits, codebook 2.  force_split != 0 sets the number of k-slices
+ * (negative, m > 128: that many, in the 256-row kernel with the fewest row tiles).  exl3_dgemm_pays: 1 if the call is faster than a rebuilt fp16 matrix and a plain GEMM, 0 if not (129 .. 1023 rows). */
 int exl3_dgemm_plan(int m, int k, int n, int* xh_rows, int64_t* slab_floats);
+int exl3_dgemm_plan_kind(int m, int k, int n, int K, int cb, int* xh_rows, int64_t* slab_floats);
+int exl3_dgemm_pays(int m, int k, int n, int K, int cb);
 int exl3_dgemm(const void* x, int64_t ldx, const void* const* suhs, void* xh, int xh_rows, const void* const* trellis, const void* const* svhs,
                const void* const* biases, void* const* Cs, const int64_t* ldcs, const int* ns, int count, int out, void* slab, int64_t slab_floats,
                int m, int k, int K, int cb, int force_split, void* stream);

@@ -200,3 +200,37 @@ def test_a_bias_of_another_form_keeps_its_route(form):
     lin = LinearEXL3(k, n, tr, su, sv, mul1=True, bias=bias)
     q, p = LinearEXL3.forward_separate([lin, LinearEXL3(k, n, tr, su, sv, mul1=True)], x)
     assert torch.equal(q, y) and _err(p, exact(x)) < 6e-4
+
+
+@pytest.mark.parametrize("k,n,rows,K,cb,packed", [
+    (4096, 6144, 560, 8, 0, False), (4096, 6144, 300, 4, 2, True), (4096, 4096, 768, 8, 0, False), (4096, 14336, 512, 4, 2, True), (4096, 14336, 600, 8, 1, False),
+    (14336, 4096, 1000, 4, 2, True), (2048, 512, 1000, 8, 0, True), (2048, 512, 1023, 4, 2, True), (2048, 512, 1024, 4, 2, False)])
+def test_route_follows_sizes_bits_and_codebook(k, n, rows, K, cb, packed):
+    """The route with the fp16 weight matrix gives the bits of the forced one, the packed one does not; points where the two are at least 5 % apart, and the last row count."""
+    from exllamav3_amd.linear import LinearEXL3
+    gen = torch.Generator(device=_dev()).manual_seed(rows + K)
+    tr = torch.randint(-32768, 32768, (k // 16, n // 16, 16 * K), dtype=torch.int16, device=_dev(), generator=gen)
+    su = (torch.randint(0, 2, (k,), device=_dev(), generator=gen) * 2 - 1).half()
+    sv = (0.02 * torch.rand(n, device=_dev(), generator=gen)).half()
+    lin = LinearEXL3(k, n, tr, su, sv, mcg=cb == 1, mul1=cb == 2)
+    x = torch.randn((rows, k), device=_dev(), generator=gen).half()
+    y, other = lin.forward(x), lin.forward(x, {"reconstruct": True})
+    assert _err(y, other.double()) < 9e-4                 # (both rounded as in the bounds above)
+    assert torch.equal(y, other) != packed
+
+
+@pytest.mark.parametrize("m", [40, 100, 144, 150, 200, 420, 700, 1000])
+@pytest.mark.parametrize("K,cb", [(3, 1), (7, 2), (8, 0)])
+def test_dgemm_full_size_plans(m, K, cb):
+    """A model's size, where plans split k and use several row tiles: against the same product with one slice, 2e-6 of the largest float32 sums of 4096 products apart."""
+    from exllamav3_amd import ext
+    k, n = 4096, 1024
+    gen = torch.Generator(device=_dev()).manual_seed(m + K)
+    tr = torch.randint(-32768, 32768, (k // 16, n // 16, 16 * K), dtype=torch.int16, device=_dev(), generator=gen)
+    su, sv = torch.ones(k, device=_dev()).half(), torch.ones(n, device=_dev()).half()
+    x = torch.randn((m, k), device=_dev(), generator=gen).half()
+    ys = [torch.full((m, n), float("nan"), device=_dev()) for _ in range(3)]
+    for y, split in zip(ys, (0, 1, -1)):
+        ext.dgemm(x, [tr], [y], [su], [sv], cb == 1, cb == 2, force_split=split)
+    for y in ys[1:]:
+        assert float((ys[0] - y).abs().max()) < 2e-6 * float(ys[0].abs().max()) * 4
