@@ -88,7 +88,8 @@ __device__ __forceinline__ void ps_st128_sys(ps_rsrc_t r, uint32_t byte_off, uin
 // each slice's contribution (2^-11 relative, like the activations the consumer forms from it).  The residual row's blocks (rbuf) stay fp32 lines.
 // A/B builds: PS_FP32_PARTIALS keeps the 1 KiB fp32 lines.
 // acc + f * (half of a pair): one mixed-precision instruction instead of a conversion and an addition (or three with a factor).  With f = 1 the product is exact: the same sum.
-// The sums of partial lines stand in every op's latency chain: two instructions per value fewer and Llama-3.2-1B's step goes from 527 to 521 us (526 at the start of these measurements with packed additions, which some forms of this hardware get wrong)
+// The sums of partial lines stand in every op's latency chain.  Two instructions per value fewer take Llama-3.2-1B's step from 527 to 521 us, with the edges of up to 16 slices (PS_COOP_MIN) to 516:
+// where it stood with packed float32 additions, some forms of which this hardware gets wrong
 __device__ __forceinline__ float ps_mix_lo(float acc, uint32_t pair, float f) { float r; asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(pair), "v"(f), "v"(acc)); return r; }
 __device__ __forceinline__ float ps_mix_hi(float acc, uint32_t pair, float f) { float r; asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(pair), "v"(f), "v"(acc)); return r; }
 __device__ __forceinline__ float ps_mix1_lo(float acc, uint32_t pair) { float r; asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(pair), "v"(acc)); return r; }
@@ -1166,8 +1167,8 @@ __global__ __launch_bounds__(PS_NT) void exl3_pstep_kernel(const PsArgs a)
             if (in_type == PS_IN_NORM && in_direct)
             {
                 // DIRECT residual edge: this workgroup finishes the blocks of ITS slice of the row's new version from the producer op's partial lines -- ONE hop
-                // (partial lines -> here) instead of two (partial lines -> owner -> owner's line -> every workgroup).  All eight service half-waves gather (half-wave h:
-                // lines h, h + 8, ... of a block, two blocks per round while S_in <= 16), the block's half-wave adds the eight sums in the owners' order, output
+                // (partial lines -> here) instead of two (partial lines -> owner -> owner's line -> every workgroup).  The block's own half-wave sums up to PS_COOP_MIN
+                // lines; of more, all eight service half-waves gather (half-wave h: lines h, h + 8, ... of a block) and the block's adds their sums in order.  Then the output
                 // Hadamard, the producer's svh, + the block of the previous version; one workgroup per slice (PS_TILE_Q_OUT) publishes the new blocks and their
                 // sums of squares.  The quads are formed with r_last; the true scale needs every block's sum of squares: see the finish below
                 if (sw == 0) PS_T(4);
@@ -1213,19 +1214,17 @@ __global__ __launch_bounds__(PS_NT) void exl3_pstep_kernel(const PsArgs a)
                 {
                     const ps_rsrc_t rp = ps_rsrc(O->in_slab[0]);
                     const int S_p = O->S_in;
-                    // NSLOT lines per half-wave and round trip: with <= 16 slices a half-wave has two lines per block -> NSLOT / 2 blocks per round (all four with the fp16
-                    // lines); with up to 32 slices four lines per block
+                    // NSLOT lines per half-wave and round trip, four per block (up to 32 slices)
 #ifndef PS_FP32_PARTIALS
                     constexpr int NSLOT = 8;
 #else
                     constexpr int NSLOT = 4;
 #endif
-                    const bool two = S_p <= 16;
-                    const int lpb = two ? 2 : 4, bpr = NSLOT / lpb;           // lines per block and half-wave, blocks per round
+                    constexpr int bpr = NSLOT / 4;                          // blocks per round
                     const int rounds = (nb + bpr - 1) / bpr;
                     for (int r = 0; r < rounds; ++r)
                     {
-                        float4_t acc[NSLOT / 2];
+                        float4_t acc[bpr];
                         for (int spins = 0;; ++spins)
                         {
                             PsPl t[NSLOT];
@@ -1233,33 +1232,28 @@ __global__ __launch_bounds__(PS_NT) void exl3_pstep_kernel(const PsArgs a)
                             #pragma unroll
                             for (int i = 0; i < NSLOT; ++i)
                             {
-                                const int jj = r * bpr + (two ? (i >> 1) : (i >> 2)), s_ = shw + 8 * (two ? (i & 1) : (i & 3));
+                                const int jj = r * bpr + (i >> 2), s_ = shw + 8 * (i & 3);
                                 t[i] = ps_pl_load_t<SYS>(rp, ((uint32_t) (b0 + min(jj, nb - 1)) * (uint32_t) S_p + (uint32_t) min(s_, S_p - 1)) * PS_PLINE_BYTES, l32);
                             }
                             #pragma unroll
-                            for (int q = 0; q < NSLOT / 2; ++q) acc[q] = float4_t{ 0.f, 0.f, 0.f, 0.f };
-                            auto take = [&] (auto twoc)
+                            for (int q = 0; q < bpr; ++q) acc[q] = float4_t{ 0.f, 0.f, 0.f, 0.f };
+                            ps_static_for<0, NSLOT>([&] (auto ic)
                             {
-                                constexpr bool TWO = decltype(twoc)::value;
-                                ps_static_for<0, NSLOT>([&] (auto ic)
-                                {
-                                    constexpr int i = decltype(ic)::value, bi = TWO ? (i >> 1) : (i >> 2);
-                                    const int jj = r * bpr + bi, s_ = shw + 8 * (TWO ? (i & 1) : (i & 3));
-                                    const bool use = jj < nb && s_ < S_p;
-                                    ok &= !use | ps_pl_ok(t[i], tag_in);
-                                    ps_pl_add(acc[bi], t[i], use ? 0xffffffffu : 0u);
-                                });
-                            };
-                            if (two) take(std::true_type{}); else take(std::false_type{});
+                                constexpr int i = decltype(ic)::value, bi = i >> 2;
+                                const int jj = r * bpr + bi, s_ = shw + 8 * (i & 3);
+                                const bool use = jj < nb && s_ < S_p;
+                                ok &= !use | ps_pl_ok(t[i], tag_in);
+                                ps_pl_add(acc[bi], t[i], use ? 0xffffffffu : 0u);
+                            });
                             if (__builtin_amdgcn_ballot_w64(!ok) == 0ull) break;
                             if (spins > slim) { ps_timeout(8u); break; }
                             __builtin_amdgcn_s_sleep(PS_POLL_SLEEP);
                         }
                         #pragma unroll
-                        for (int q = 0; q < NSLOT / 2; ++q)
+                        for (int q = 0; q < bpr; ++q)
                         {
                             const int jj = r * bpr + q;
-                            if (q < bpr && jj < nb) ((float4_t*) (gath + ((size_t) (jj & 3) * 8 + shw) * 128))[l32] = acc[q];
+                            if (jj < nb) ((float4_t*) (gath + ((size_t) (jj & 3) * 8 + shw) * 128))[l32] = acc[q];
                         }
                     }
                     tgt_o += PS_NSV;
