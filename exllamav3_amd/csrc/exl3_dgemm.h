@@ -1,6 +1,7 @@
 // Arguments and the output stage of exl3_dgemm (medium row counts), shared by the kernel units (one per bits-per-weight) and the launcher.
 #pragma once
 #include "exl3_common.cuh"
+#include <atomic>
 #include <type_traits>
 
 #define DG_PITCH 136            // floats per row of the output tile in LDS: row groups 0 | 1 (and 2 | 3) of an accumulator touch different banks
@@ -211,4 +212,18 @@ __device__ __forceinline__ void dg_epilogue(const DgemmArgs& a, const DgTile& t,
         const float4_t h = { __builtin_fmaf(y.x, sgn, x.x), __builtin_fmaf(y.y, sgn, x.y), __builtin_fmaf(y.z, sgn, x.z), __builtin_fmaf(y.w, sgn, x.w) };
         if (t.row0 + row < t.row_end) dg_put(a, t.C, (int64_t) (t.row0 + row) * t.ldc + t.cb * 128 + 4 * l, h, f, bv);
     }
+}
+
+// Launch of one of the kernels.  More than 64 KB of LDS per workgroup (the narrow kernel's 128-row form, the wide one's all) is asked for once per kernel and device, in front of the first launch there.
+template <void (*KERNEL)(const DgemmArgs)>
+static void dg_start(dim3 grid, size_t lds, hipStream_t st, const DgemmArgs& a)
+{
+    static std::atomic<uint64_t> ready{ 0 };
+    int dev = 0;
+    if (lds > 65536 && hipGetDevice(&dev) == hipSuccess && !((ready.load(std::memory_order_relaxed) >> (dev & 63)) & 1))
+    {
+        (void) hipFuncSetAttribute((const void*) KERNEL, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds);
+        ready.fetch_or(1ull << (dev & 63), std::memory_order_relaxed);
+    }
+    KERNEL<<<grid, dim3(256), lds, st>>>(a);
 }

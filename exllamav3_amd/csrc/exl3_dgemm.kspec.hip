@@ -151,7 +151,7 @@ static void dg_launch_cb(int mt, dim3 grid, size_t lds, hipStream_t st, const Dg
 {
     switch (mt)
     {
-        #define DG(M) case M: exl3_dgemm_kernel<G2_K, CB, M><<<grid, dim3(256), lds, st>>>(a); break;
+        #define DG(M) case M: dg_start<exl3_dgemm_kernel<G2_K, CB, M>>(grid, lds, st, a); break;
         DG(4) DG(5) DG(6) DG(7) DG(8)
         #undef DG
     }

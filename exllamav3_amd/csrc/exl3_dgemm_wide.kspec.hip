@@ -13,7 +13,6 @@
 #include "exl3_api_internal.h"
 #include "exl3_lane_decode.cuh"
 #include "exl3_dgemm.h"
-#include <atomic>
 
 __device__ __forceinline__ void dg_mfma(float4_t& acc, const half8_t& a, const half8_t& b)
 {
@@ -167,27 +166,12 @@ void exl3_dgemm_wide_kernel(const DgemmArgs a)
 #error "compile with -DG2_K=<bits per weight>"
 #endif
 
-// (more than 64 KB of LDS per workgroup is a property of the kernel on a device, set in front of its first launch there)
-template <int CB, int MT>
-static void dgw_launch(dim3 grid, size_t lds, hipStream_t st, const DgemmArgs& a)
-{
-    static std::atomic<uint64_t> ready{ 0 };
-    int dev = 0;
-    (void) hipGetDevice(&dev);
-    if (!((ready.load(std::memory_order_relaxed) >> (dev & 63)) & 1))
-    {
-        (void) hipFuncSetAttribute((const void*) exl3_dgemm_wide_kernel<G2_K, CB, MT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds);
-        ready.fetch_or(1ull << (dev & 63), std::memory_order_relaxed);
-    }
-    exl3_dgemm_wide_kernel<G2_K, CB, MT><<<grid, dim3(256), lds, st>>>(a);
-}
-
 template <int CB>
 static void dgw_launch_cb(int mt, dim3 grid, size_t lds, hipStream_t st, const DgemmArgs& a)
 {
     switch (mt)
     {
-        #define DG(M) case M: dgw_launch<CB, M>(grid, lds, st, a); break;
+        #define DG(M) case M: dg_start<exl3_dgemm_wide_kernel<G2_K, CB, M>>(grid, lds, st, a); break;
         DG(10) DG(12) DG(14) DG(16)
         #undef DG
     }
