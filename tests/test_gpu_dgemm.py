@@ -234,3 +234,22 @@ def test_dgemm_full_size_plans(m, K, cb):
         ext.dgemm(x, [tr], [y], [su], [sv], cb == 1, cb == 2, force_split=split)
     for y in ys[1:]:
         assert float((ys[0] - y).abs().max()) < 2e-6 * float(ys[0].abs().max()) * 4
+
+
+@pytest.mark.parametrize("rows", [150, 256, 300, 500])
+def test_gate_and_up_of_a_models_size(rows):
+    """Both matrices of one launch with the activation behind it where the GEMM's fused epilogue ran from 256 rows on: against the two linears through rebuilt weights."""
+    from exllamav3_amd import ext
+    from exllamav3_amd.linear import LinearEXL3, _dgemm_ok
+    k, n, K = 4096, 8192, 4
+    gen = torch.Generator(device=_dev()).manual_seed(rows)
+
+    def lin():
+        tr = torch.randint(-32768, 32768, (k // 16, n // 16, 16 * K), dtype=torch.int16, device=_dev(), generator=gen)
+        return LinearEXL3(k, n, tr, (torch.randint(0, 2, (k,), device=_dev(), generator=gen) * 2 - 1).half(), (0.02 * torch.rand(n, device=_dev(), generator=gen)).half(), mul1=True)
+    gate, up = lin(), lin()
+    x = torch.randn((rows, k), device=_dev(), generator=gen).half()
+    assert _dgemm_ok(x, (gate, up), rows)
+    g, u = (l.forward(x, {"reconstruct": True}).double() for l in (gate, up))
+    # (gate and up: rotated rows against W^T, rounded to fp16 on both sides; the activation rounded once: five errors of 2.8e-4, and silu's slope of up to 1.1)
+    assert _err(LinearEXL3.forward_gate_up_silu(gate, up, x), torch.nn.functional.silu(g) * u) < 8e-4

@@ -58,3 +58,19 @@ def test_block_on_packed_weights_matches_the_loop_over_experts(dev, T):
     again = moe.forward_prefill(row)
     keep = torch.arange(T, device=dev) != 7
     assert again[7].isnan().all() and torch.equal(again[keep], got[keep])
+
+
+@pytest.mark.parametrize("T", [130, 1100, 2560])
+def test_block_of_a_models_size_on_packed_weights(dev, T):
+    """Mixtral's block over the chunks that take the packed form, against the form on rebuilt weights.  Bound: in each of the two products one side rounds the rotated rows and the other W^T, the
+    activations between them are rounded on both: six errors of 2^-11 / sqrt(3) at most, 7e-4 together; no row of a token may be further off than three times that."""
+    from exllamav3_amd.moe_path import SyntheticEXL3MoE
+    moe = SyntheticEXL3MoE(4096, 14336, experts=8, top_k=2, K=4, cb=2, device=dev, seed=11)
+    moe.router.copy_(torch.randn(moe.router.shape, device=dev, generator=torch.Generator(device=dev).manual_seed(3)) / 64)
+    x = torch.randn((T, 4096), device=dev, generator=torch.Generator(device=dev).manual_seed(5)).half()
+    assert moe._on_packed_weights(2 * T)
+    got = moe.forward_prefill(x)
+    moe.DGEMM_ROWS = 0
+    want = moe.forward_prefill(x)
+    assert (got - want).norm() / want.norm() < 8e-4
+    assert float(((got - want).norm(dim=1) / want.norm(dim=1)).max()) < 2.4e-3
