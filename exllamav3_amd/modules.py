@@ -155,6 +155,7 @@ class GatedLinearAttention:
     # key dimensions whose segments run in chunks of 16 rows: a workgroup covers 128 value columns and two of them fill a compute unit, and even one segment is faster than
     # the row-by-row chain (16 heads of 64 x 128, us: 2048 rows 2130 as a chain, 738 as one segment, 78 as 16; 5 x 256 rows 266, 105, 50 as 6; 300 + 200 rows 310, 119, 39 as 7)
     CHUNK_DIMS, CHUNK_MIN_ROWS, CHUNK_TARGET_WORKGROUPS = (64, 128), 48, 512
+    a2 = None                     # the decay's second matrix, once weights are loaded (its columns are the rank)
 
     def __init__(self, width: int, heads: int, dim: int, vdim: int, tau: float, eps: float):
         self.width, self.heads, self.dim, self.vdim, self.tau, self.eps = width, heads, dim, vdim, float(tau), float(eps)
@@ -176,7 +177,7 @@ class GatedLinearAttention:
 
     def segments(self, sb: StepBatch) -> tuple[int, int] | None:
         """(segments per sequence, rows per segment) for a long prompt step: enough workgroups to fill the device, segments of at least 64 rows (48 in chunks)."""
-        if self.dim in self.CHUNK_DIMS and self.a2.shape[1] <= 64:
+        if self.dim in self.CHUNK_DIMS and (self.a2 is None or self.a2.shape[1] <= 64):
             if sb.max_rows < self.CHUNK_MIN_ROWS:
                 return None
             chains = sb.batch * self.heads * ((self.vdim + 127) // 128)

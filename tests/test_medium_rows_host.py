@@ -37,3 +37,17 @@ def test_rule_and_entry_point_agree_on_the_largest_call(groups, k):
         assert rc < 0 and (b"below 2 GiB" in text or b"aligned outputs" in text), text
         return b"below 2 GiB" in text
     assert not refused(lo) and refused(hi)
+
+
+def test_segments_of_a_layer_without_weights():
+    """The cut of a prompt into segments is asked of a layer by its sizes alone (the benchmark of the mixer families does)."""
+    import torch
+    from exllamav3_amd.modules import GatedLinearAttention
+    from exllamav3_amd.state_cache import StepBatch
+    none = torch.zeros(1, dtype=torch.int32)
+    step = lambda rows: StepBatch(rows, 1, False, rows, None, none, none, none, none, none, none)
+    for dim, least in ((64, 48), (128, 48), (96, 256)):
+        layer = GatedLinearAttention(2048, 16, dim, 128, 16.0, 1e-5)
+        assert layer.segments(step(least - 1)) is None
+        segs, length = layer.segments(step(4096))
+        assert segs >= 2 and segs * length >= 4096 and (dim == 96 or length % 16 == 0)
