@@ -29,7 +29,7 @@ template <typename T> __host__ __device__ constexpr int wide_n() { return 16 / (
 #define ROW_HELD 4
 
 // h = x inv w for the row whose first pieces are in `held`; the others come from x, which the same thread wrote or read
-template <typename T, int V>
+template <typename T, int V, int NT = ROW_THREADS>
 __device__ __forceinline__ void row_norm_write(T* __restrict__ hr, const float* xr, const float* __restrict__ w, const float (&held)[ROW_HELD][V], float inv, int width)
 {
     auto write = [&] (int i, const float (&v)[V]) __attribute__((always_inline))
@@ -41,8 +41,8 @@ __device__ __forceinline__ void row_norm_write(T* __restrict__ hr, const float* 
         store_n<T, V>(hr + i, wv);
     };
     #pragma unroll
-    for (int u = 0; u < ROW_HELD; ++u) { const int i = (u * ROW_THREADS + threadIdx.x) * V; if (i < width) write(i, held[u]); }
-    for (int i = (ROW_HELD * ROW_THREADS + threadIdx.x) * V; i < width; i += ROW_THREADS * V) { float t[V]; load_n<float, V>(xr + i, t); write(i, t); }
+    for (int u = 0; u < ROW_HELD; ++u) { const int i = (u * NT + threadIdx.x) * V; if (i < width) write(i, held[u]); }
+    for (int i = (ROW_HELD * NT + threadIdx.x) * V; i < width; i += NT * V) { float t[V]; load_n<float, V>(xr + i, t); write(i, t); }
 }
 
 template <typename T, int V>
@@ -105,11 +105,12 @@ __global__ __launch_bounds__(ROW_THREADS) void rms_norm_rows_kernel(T* __restric
     row_norm_write<T, V>(h + (int64_t) n * width, xr, w, held, inv, width);
 }
 
-template <typename T, int V>
-__global__ __launch_bounds__(ROW_THREADS) void gated_residual_kernel(float* __restrict__ x, const T* __restrict__ y, int64_t y_ld, const T* __restrict__ r,
+template <typename T, int V, int NW>
+__global__ __launch_bounds__(64 * NW) void gated_residual_kernel(float* __restrict__ x, const T* __restrict__ y, int64_t y_ld, const T* __restrict__ r,
                                                                      int64_t r_ld, const float* __restrict__ norm_w, T* __restrict__ h, float eps, int width)
 {
-    __shared__ float red[ROW_WAVES];
+    constexpr int NT = 64 * NW;
+    __shared__ float red[NW];
     const int n = blockIdx.x;
     float* xr = x + (int64_t) n * width;
     const T* yr = y + (int64_t) n * y_ld;
@@ -125,30 +126,29 @@ __global__ __launch_bounds__(ROW_THREADS) void gated_residual_kernel(float* __re
     #pragma unroll
     for (int u = 0; u < ROW_HELD; ++u)
     {
-        const int i = (u * ROW_THREADS + threadIdx.x) * V;
+        const int i = (u * NT + threadIdx.x) * V;
         if (i < width) { load_n<float, V>(xr + i, held[u]); load_n<T, V>(yr + i, yv[u]); load_n<T, V>(rr + i, rv[u]); }
     }
     #pragma unroll
-    for (int u = 0; u < ROW_HELD; ++u) { const int i = (u * ROW_THREADS + threadIdx.x) * V; if (i < width) form(i, held[u], yv[u], rv[u]); }
-    for (int i = (ROW_HELD * ROW_THREADS + threadIdx.x) * V; i < width; i += ROW_THREADS * V)
+    for (int u = 0; u < ROW_HELD; ++u) { const int i = (u * NT + threadIdx.x) * V; if (i < width) form(i, held[u], yv[u], rv[u]); }
+    for (int i = (ROW_HELD * NT + threadIdx.x) * V; i < width; i += NT * V)
     {
         float v[V], a[V], g[V];
         load_n<float, V>(xr + i, v); load_n<T, V>(yr + i, a); load_n<T, V>(rr + i, g);
         form(i, v, a, g);
     }
     if (!norm_w) return;
-    ss = block_sum<ROW_WAVES>(ss, red);
+    ss = block_sum<NW>(ss, red);
     const float inv = 1.0f / sqrtf(ss / (float) width + eps);
-    row_norm_write<T, V>(h + (int64_t) n * width, xr, norm_w, held, inv, width);
+    row_norm_write<T, V, NT>(h + (int64_t) n * width, xr, norm_w, held, inv, width);
 }
 
-#define POLY_WAVES 8
-template <typename T, int V>
-__global__ __launch_bounds__(64 * POLY_WAVES) void polynorm_kernel(T* __restrict__ out, const T* __restrict__ z, int64_t z_ld, const float* __restrict__ coef,
+template <typename T, int V, int NW>
+__global__ __launch_bounds__(64 * NW) void polynorm_kernel(T* __restrict__ out, const T* __restrict__ z, int64_t z_ld, const float* __restrict__ coef,
                                                                    float eps, int ff)
 {
-    constexpr int NT = 64 * POLY_WAVES;
-    __shared__ float red[3][POLY_WAVES];
+    constexpr int NT = 64 * NW;
+    __shared__ float red[3][NW];
     const int n = blockIdx.x;
     const T* zr = z + (int64_t) n * z_ld;
     float held[ROW_HELD][V];
@@ -172,7 +172,7 @@ __global__ __launch_bounds__(64 * POLY_WAVES) void polynorm_kernel(T* __restrict
     __syncthreads();
     s1 = s2 = s3 = 0.f;
     #pragma unroll
-    for (int i = 0; i < POLY_WAVES; ++i) { s1 += red[0][i]; s2 += red[1][i]; s3 += red[2][i]; }
+    for (int i = 0; i < NW; ++i) { s1 += red[0][i]; s2 += red[1][i]; s3 += red[2][i]; }
     const float i1 = 1.0f / sqrtf(s1 / (float) ff + eps), i2 = 1.0f / sqrtf(s2 / (float) ff + eps), i3 = 1.0f / sqrtf(s3 / (float) ff + eps);
     const float a = coef[0], b = coef[1], c = coef[2], k = coef[3];
     T* o = out + (int64_t) n * ff;
@@ -243,8 +243,9 @@ extern "C" int exl3_mix_gated_residual(float* x, const void* y, int64_t y_ld, co
 {
     MIX_CHECK(x && y && r && n >= 0 && width > 0 && y_ld >= width && r_ld >= width && (!norm_w || h), "mix_gated_residual: bad arguments");
     if (n == 0) return EXL3_MIX_OK;
-    #define GATED(VV) hipLaunchKernelGGL((gated_residual_kernel<T, VV>), dim3(n), dim3(ROW_THREADS), 0, (hipStream_t) stream, x, (const T*) y, y_ld, (const T*) r, r_ld, norm_w, (T*) h, eps, width)
-    MIX_DISPATCH_T(dtype, if (row_wide<T>(width, y_ld) && row_wide<T>(width, r_ld) && aligned16(x, y, r, norm_w) && aligned16(h, nullptr, nullptr, nullptr)) GATED(wide_n<T>()); else GATED(1));
+    // (1000 wide, 4096 rows of bfloat16: 14.4 us with four waves, 11.6 with the two that the row keeps busy)
+    #define GATED(VV, NW) hipLaunchKernelGGL((gated_residual_kernel<T, VV, NW>), dim3(n), dim3(64 * NW), 0, (hipStream_t) stream, x, (const T*) y, y_ld, (const T*) r, r_ld, norm_w, (T*) h, eps, width)
+    MIX_DISPATCH_T(dtype, if (row_wide<T>(width, y_ld) && row_wide<T>(width, r_ld) && aligned16(x, y, r, norm_w) && aligned16(h, nullptr, nullptr, nullptr)) { if (width <= 128 * wide_n<T>()) GATED(wide_n<T>(), 2); else GATED(wide_n<T>(), 4); } else GATED(1, 4));
     #undef GATED
     return mix_check_launch("mix_gated_residual");
 }
@@ -253,8 +254,10 @@ extern "C" int exl3_mix_polynorm(void* out, const void* z, int64_t z_ld, const f
 {
     MIX_CHECK(out && z && coef && n >= 0 && ff > 0 && z_ld >= ff, "mix_polynorm: bad arguments");
     if (n == 0) return EXL3_MIX_OK;
-    #define POLY(VV) hipLaunchKernelGGL((polynorm_kernel<T, VV>), dim3(n), dim3(64 * POLY_WAVES), 0, (hipStream_t) stream, (T*) out, (const T*) z, z_ld, coef, eps, ff)
-    MIX_DISPATCH_T(dtype, if (row_wide<T>(ff, z_ld) && aligned16(out, z, nullptr, nullptr)) POLY(wide_n<T>()); else POLY(1));
+    // waves that a row keeps busy (bfloat16, 4096 rows, us with 8 waves / here: 1000 wide 14.9 / 7.3, 2048 wide 17.4 / 11.6; single elements, 2050 wide 17.6 / 14.7)
+    #define POLY(VV, NW) hipLaunchKernelGGL((polynorm_kernel<T, VV, NW>), dim3(n), dim3(64 * NW), 0, (hipStream_t) stream, (T*) out, (const T*) z, z_ld, coef, eps, ff)
+    MIX_DISPATCH_T(dtype, constexpr int V = wide_n<T>(); if (!row_wide<T>(ff, z_ld) || !aligned16(out, z, nullptr, nullptr)) POLY(1, 4); else if (ff <= 128 * V) POLY(V, 2);
+                          else if (ff <= 256 * V) POLY(V, 4); else POLY(V, 8));
     #undef POLY
     return mix_check_launch("mix_polynorm");
 }

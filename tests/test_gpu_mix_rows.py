@@ -50,6 +50,12 @@ def test_norms_and_gates(width, off, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("width,off", [(512, 0), (516, 0), (1000, 0), (1032, 0), (2048, 0), (2050, 0)])
+def test_norms_and_gates_at_the_widths_where_the_waves_change(width, off, dtype):
+    test_norms_and_gates(width, off, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("vdim,heads,off", [(4, 3, 0), (33, 2, 0), (64, 5, 0), (128, 32, 0), (128, 3, 2), (132, 1, 0), (256, 2, 4), (300, 2, 0)])
 def test_gla_out(vdim, heads, off, dtype):
     from exllamav3_amd import mix_ops
