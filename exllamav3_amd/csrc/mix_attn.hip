@@ -40,8 +40,8 @@ __global__ __launch_bounds__(64) void attn_store_kernel(T* __restrict__ v_norm, 
 // the values of the head's key/value head, and the result is [row][head][map][vdim].  mask 0: the last `window` positions; 1: the positions of the row's
 // own chunk of `window` positions (a chunk starts where the position is a multiple of `window`).  keep: the first `keep` positions stay visible whatever the mask
 // says.  gate: one number per head (gate_cols 1) or one per value element (gate_cols vdim).
-template <typename T, int MAXV, typename TO, int NW>
-__global__ __launch_bounds__(64 * NW) void attn_prefill_kernel(TO* __restrict__ out, int64_t out_ld, const T* __restrict__ q, int64_t q_ld, const T* __restrict__ k, int64_t k_ld,
+template <typename T, int MAXV, typename TO>
+__global__ __launch_bounds__(64 * AT_WAVES) void attn_prefill_kernel(TO* __restrict__ out, int64_t out_ld, const T* __restrict__ q, int64_t q_ld, const T* __restrict__ k, int64_t k_ld,
                                                           const T* __restrict__ v, int64_t v_ld, const T* __restrict__ gate, int64_t gate_ld, int gate_cols, const float* __restrict__ sink,
                                                           const int32_t* __restrict__ cu, const int32_t* __restrict__ tok_seq, const int32_t* __restrict__ tok_pos,
                                                           int heads, int kv_heads, int maps, int dim, int vdim, float scale, float softcap, int window, int mask, int keep, float out_scale)
@@ -59,20 +59,20 @@ __global__ __launch_bounds__(64 * NW) void attn_prefill_kernel(TO* __restrict__ 
     {
         const int kept = min(keep, lo);
         const T* k0 = k + (int64_t) first * k_ld + (int64_t) kh * dim;
-        attn_row<T, MAXV, TO, NW, row_jump>(out + (int64_t) n * out_ld + (int64_t) h * vdim, q + (int64_t) n * q_ld + (int64_t) h * dim, q, dim, k0, k_ld,
+        attn_row<T, MAXV, false, TO, AT_WAVES, row_jump>(out + (int64_t) n * out_ld + (int64_t) h * vdim, q + (int64_t) n * q_ld + (int64_t) h * dim, q, dim, k0, k_ld,
                               v + (int64_t) first * v_ld + (int64_t) g * vdim, v_ld, kept + i - lo + 1, dim, vdim, scale, sink != nullptr, sink ? sink[h] : 0.f, gt,
                               rows_are_16_byte(k0, k_ld, dim), smem, softcap, row_jump{kept, (int64_t) (lo - kept)}, grow);
         return;
     }
     const T* kb = k + (int64_t) (first + lo) * k_ld + (int64_t) kh * dim;
-    attn_row<T, MAXV, TO, NW>(out + (int64_t) n * out_ld + (int64_t) h * vdim, q + (int64_t) n * q_ld + (int64_t) h * dim, q, dim, kb, k_ld,
+    attn_row<T, MAXV, false, TO, AT_WAVES>(out + (int64_t) n * out_ld + (int64_t) h * vdim, q + (int64_t) n * q_ld + (int64_t) h * dim, q, dim, kb, k_ld,
                           v + (int64_t) (first + lo) * v_ld + (int64_t) g * vdim, v_ld,
                           i - lo + 1, dim, vdim, scale, sink != nullptr, sink ? sink[h] : 0.f, gt, rows_are_16_byte(kb, k_ld, dim), smem, softcap, row_linear(), grow);
 }
 
 // Rings: ring_k [slots][window][kv_heads * maps][dim], ring_v [slots][window][kv_heads][vdim], entry = position % window.  mask 0: the newest
 // min(len, window) entries (all of them, in any order); 1: the row's chunk, which is the entries 0 .. (len - 1) % window.
-template <typename T, int MAXV, typename TO, int NW>
+template <typename T, int MAXV, bool LINES, typename TO, int NW>
 __global__ __launch_bounds__(64 * NW) void attn_decode_kernel(TO* __restrict__ out, int64_t out_ld, const T* __restrict__ q, int64_t q_ld, const T* __restrict__ ring_k,
                                                          const T* __restrict__ ring_v, const T* __restrict__ gate, int64_t gate_ld, int gate_cols, const float* __restrict__ sink,
                                                          const int32_t* __restrict__ slots, const int32_t* __restrict__ len_after,
@@ -88,7 +88,7 @@ __global__ __launch_bounds__(64 * NW) void attn_decode_kernel(TO* __restrict__ o
     const float gt = by_head ? sigmoid_f(to_f(gate[(int64_t) n * gate_ld + h])) * out_scale : out_scale;
     const T* grow = gate && !by_head ? gate + (int64_t) n * gate_ld + (int64_t) h * vdim : nullptr;
     const T* kb = ring_k + (row0 * kheads + kh) * dim;
-    attn_row<T, MAXV, TO, NW>(out + (int64_t) n * out_ld + (int64_t) h * vdim, q + (int64_t) n * q_ld + (int64_t) h * dim, q, dim,
+    attn_row<T, MAXV, LINES, TO, NW>(out + (int64_t) n * out_ld + (int64_t) h * vdim, q + (int64_t) n * q_ld + (int64_t) h * dim, q, dim,
                           kb, (int64_t) kheads * dim, ring_v + (row0 * kv_heads + g) * vdim, (int64_t) kv_heads * vdim,
                           count, dim, vdim, scale, sink != nullptr, sink ? sink[h] : 0.f, gt, rows_are_16_byte(kb, (int64_t) kheads * dim, dim), smem, softcap, row_linear(), grow);
 }
@@ -106,24 +106,20 @@ extern "C" int exl3_mix_attn_store(void* v_norm, void* ring_k, void* ring_v, con
     return mix_check_launch("mix_attn_store");
 }
 
-#define ATTN_LAUNCH_NW(KERNEL, TO, NWV, ...) \
-    do { \
-        const size_t sm = (size_t) (dim + NWV * 64 + NWV * (2 + mvt * 64)) * sizeof(float); \
-        if (mv == 1)      hipLaunchKernelGGL((KERNEL<T, 1, TO, NWV>), dim3(n, heads * maps), dim3(64 * NWV), sm, (hipStream_t) stream, (TO*) out, __VA_ARGS__); \
-        else if (mv == 2) hipLaunchKernelGGL((KERNEL<T, 2, TO, NWV>), dim3(n, heads * maps), dim3(64 * NWV), sm, (hipStream_t) stream, (TO*) out, __VA_ARGS__); \
-        else if (mv <= 4) hipLaunchKernelGGL((KERNEL<T, 4, TO, NWV>), dim3(n, heads * maps), dim3(64 * NWV), sm, (hipStream_t) stream, (TO*) out, __VA_ARGS__); \
-        else              hipLaunchKernelGGL((KERNEL<T, 8, TO, NWV>), dim3(n, heads * maps), dim3(64 * NWV), sm, (hipStream_t) stream, (TO*) out, __VA_ARGS__); \
-    } while (0)
-// `wide`: sixteen waves per (row, head) instead of four -- steps of few rows over long caches are bound by the chain of key chunks a wave walks, not by bytes
-#define ATTN_LAUNCH_TO(KERNEL, TO, ...) \
-    do { if (wide) ATTN_LAUNCH_NW(KERNEL, TO, 16, __VA_ARGS__); else ATTN_LAUNCH_NW(KERNEL, TO, AT_WAVES, __VA_ARGS__); } while (0)
-// the result in the activation type, or (out_f32) in float32
-#define ATTN_LAUNCH(KERNEL, ...) \
+// the kernel for vdim, with the result in the activation type or (out_f32) in float32; KERNEL(MV, TO) names an instance, NW its waves
+#define ATTN_LAUNCH_TO(KERNEL, TO, NW, ...) \
     do { \
         const int mv = (vdim + 63) / 64; \
         const int mvt = mv == 1 ? 1 : (mv == 2 ? 2 : (mv <= 4 ? 4 : 8)); \
-        MIX_DISPATCH_T(dtype, if (out_f32) ATTN_LAUNCH_TO(KERNEL, float, __VA_ARGS__); else ATTN_LAUNCH_TO(KERNEL, T, __VA_ARGS__)); \
+        const size_t sm = (size_t) (dim + NW * 64 + NW * (2 + mvt * 64)) * sizeof(float); \
+        const dim3 grid(n, heads * maps), block(64 * NW); \
+        if (mv == 1)      hipLaunchKernelGGL((KERNEL(1, TO)), grid, block, sm, (hipStream_t) stream, (TO*) out, __VA_ARGS__); \
+        else if (mv == 2) hipLaunchKernelGGL((KERNEL(2, TO)), grid, block, sm, (hipStream_t) stream, (TO*) out, __VA_ARGS__); \
+        else if (mv <= 4) hipLaunchKernelGGL((KERNEL(4, TO)), grid, block, sm, (hipStream_t) stream, (TO*) out, __VA_ARGS__); \
+        else              hipLaunchKernelGGL((KERNEL(8, TO)), grid, block, sm, (hipStream_t) stream, (TO*) out, __VA_ARGS__); \
     } while (0)
+#define ATTN_LAUNCH(KERNEL, NW, ...) \
+    do { if (out_f32) ATTN_LAUNCH_TO(KERNEL, float, NW, __VA_ARGS__); else ATTN_LAUNCH_TO(KERNEL, T, NW, __VA_ARGS__); } while (0)
 
 static int attn_check(const char* what, int n, int heads, int kv_heads, int maps, int dim, int vdim, int window, int mask, float softcap, const void* gate, int gate_cols,
                       int64_t gate_ld, int64_t out_ld)
@@ -147,9 +143,10 @@ extern "C" int exl3_mix_attn_prefill_ex(void* out, int64_t out_ld, int out_f32, 
               "mix_attn_prefill: bad row strides");
     MIX_CHECK(keep >= 0 && (keep == 0 || mask == EXL3_MIX_MASK_WINDOW), "mix_attn_prefill: kept first tokens go with a window");
     if (n == 0) return EXL3_MIX_OK;
-    const bool wide = false;
-    ATTN_LAUNCH(attn_prefill_kernel, out_ld, (const T*) q, q_ld, (const T*) k, k_ld, (const T*) v, v_ld, (const T*) gate, gate_ld, gate_cols, sink, cu, tok_seq, tok_pos,
-                heads, kv_heads, maps, dim, vdim, scale, softcap, window, mask, keep, out_scale);
+    #define PREFILL(MV, TO) attn_prefill_kernel<T, MV, TO>
+    MIX_DISPATCH_T(dtype, ATTN_LAUNCH(PREFILL, AT_WAVES, out_ld, (const T*) q, q_ld, (const T*) k, k_ld, (const T*) v, v_ld, (const T*) gate, gate_ld, gate_cols, sink, cu, tok_seq, tok_pos,
+                                      heads, kv_heads, maps, dim, vdim, scale, softcap, window, mask, keep, out_scale));
+    #undef PREFILL
     return mix_check_launch("mix_attn_prefill");
 }
 
@@ -169,9 +166,22 @@ extern "C" int exl3_mix_attn_decode_ex(void* out, int64_t out_ld, int out_f32, c
     if (int rc = attn_check("mix_attn_decode", n, heads, kv_heads, maps, dim, vdim, window, mask, softcap, gate, gate_cols, gate_ld, out_ld)) return rc;
     MIX_CHECK(q_ld >= (int64_t) heads * maps * dim, "mix_attn_decode: bad row strides");
     if (n == 0) return EXL3_MIX_OK;
+    // sixteen waves per (row, head) instead of four: steps of few rows over long caches are bound by the chain of key chunks a wave walks, not by bytes
     const bool wide = (int64_t) n * heads * maps <= 256 && window > 256 && vdim <= 256;
-    ATTN_LAUNCH(attn_decode_kernel, out_ld, (const T*) q, q_ld, (const T*) ring_k, (const T*) ring_v, (const T*) gate, gate_ld, gate_cols, sink, slots, len_after,
-                heads, kv_heads, maps, dim, vdim, scale, softcap, window, mask, out_scale);
+    const bool lines = dtype == EXL3_MIX_BF16 && rows_of_lines(ring_k, (int64_t) kv_heads * maps * dim, ring_v, (int64_t) kv_heads * vdim, dim, vdim);
+    #define DECODE_ARGS out_ld, (const T*) q, q_ld, (const T*) ring_k, (const T*) ring_v, (const T*) gate, gate_ld, gate_cols, sink, slots, len_after, \
+                        heads, kv_heads, maps, dim, vdim, scale, softcap, window, mask, out_scale
+    #define DECODE_LINES_16(MV, TO) attn_decode_kernel<T, MV, MV <= 4, TO, 16>
+    #define DECODE_LINES(MV, TO) attn_decode_kernel<T, MV, MV <= 4, TO, AT_WAVES>
+    #define DECODE_16(MV, TO) attn_decode_kernel<T, MV, false, TO, 16>
+    #define DECODE(MV, TO) attn_decode_kernel<T, MV, false, TO, AT_WAVES>
+    if (lines) { using T = bf16_t; if (wide) ATTN_LAUNCH(DECODE_LINES_16, 16, DECODE_ARGS); else ATTN_LAUNCH(DECODE_LINES, AT_WAVES, DECODE_ARGS); }
+    else MIX_DISPATCH_T(dtype, if (wide) ATTN_LAUNCH(DECODE_16, 16, DECODE_ARGS); else ATTN_LAUNCH(DECODE, AT_WAVES, DECODE_ARGS));
+    #undef DECODE
+    #undef DECODE_16
+    #undef DECODE_LINES
+    #undef DECODE_LINES_16
+    #undef DECODE_ARGS
     return mix_check_launch("mix_attn_decode");
 }
 

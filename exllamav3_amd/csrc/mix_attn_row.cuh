@@ -12,6 +12,12 @@
 // TO: the element type of the result (float keeps the weighted sum unrounded for a caller that combines several maps).
 #define AT_WAVES 4
 
+// Whether bfloat16 rows take the form that reads whole 128-byte lines: rows of 64, 128, .. elements at addresses of 16 bytes, values of at most 256 (the accumulators fit)
+static inline bool rows_of_lines(const void* k, int64_t k_step, const void* v, int64_t v_step, int dim, int vdim)
+{
+    return dim % 64 == 0 && vdim % 64 == 0 && vdim <= 256 && (((uintptr_t) k | (uintptr_t) v) & 15) == 0 && k_step % 8 == 0 && v_step % 8 == 0 && k_step < (1 << 27) && v_step < (1 << 27);
+}
+
 template <typename T> struct kvec;
 template <> struct kvec<bf16_t> { static constexpr int N = 8; };
 template <> struct kvec<float> { static constexpr int N = 4; };
@@ -66,7 +72,7 @@ __device__ __forceinline__ void attn_row_merge(TO* __restrict__ out, int vdim, f
     }
 }
 
-template <typename T, int MAXV, typename TO = T, int NW = AT_WAVES, typename RowMap = row_linear>
+template <typename T, int MAXV, bool LINES, typename TO = T, int NW = AT_WAVES, typename RowMap = row_linear>
 __device__ __forceinline__ void attn_row(TO* __restrict__ out, const T* __restrict__ q, const T* q2, int dim1, const T* __restrict__ kb, int64_t k_step, const T* __restrict__ vb,
                                          int64_t v_step, int count, int dim, int vdim, float scale, bool has_sink, float sink, float gate, bool k_vec,
                                          float* smem, float softcap = 0.f, RowMap map = RowMap(), const T* gate_row = nullptr)
@@ -84,108 +90,120 @@ __device__ __forceinline__ void attn_row(TO* __restrict__ out, const T* __restri
     for (int i = 0; i < MAXV; ++i) acc[i] = 0.f;
     float* pw = ps + w * 64;
     constexpr int VN = kvec<T>::N;
-    // Rows of whole 128-byte lines in bfloat16 (MAXV <= 4: the accumulators fit): eight lanes share a row, 16 bytes each, so a load instruction reads eight rows as they lie in memory
-    // -- one key per lane fetches every line eight times, and value rows two bytes at a time take 64 instructions -- and a chunk's 64 key rows and 64 value rows are all in flight
-    // at once.  Scores are added over the eight lanes, outputs over the eight rows at the end.  8 rows of 32 heads over 1000 keys of 64 dimensions: 18.4 -> 13.6 us
-    if constexpr (sizeof(T) == 2 && MAXV <= 4)
+    // LINES (rows_of_lines above): eight lanes share a row, 16 bytes each, so a load instruction reads eight rows as they lie in memory -- one key per lane fetches every
+    // line eight times, and value rows two bytes at a time take 64 instructions -- and a chunk's key rows and value rows are all in flight at once.  Scores are added over
+    // the eight lanes, outputs over the eight rows at the end.  Decode only: a kernel that held both forms spilled and ran short rows up to 1.5 times longer, and prompt
+    // rows, whose neighbours read the same keys from the caches, are faster one key per lane (200 rows of 32 heads, 128 dimensions: 45 us against 77).
+    // 8 rows of 32 heads, one key per lane / here: 1000 keys of 64 dimensions 13.6 / 10.9 us, of 128 21.0 / 15.5, of 256 66.7 / 27.1; 64 keys of 128 10.2 / 8.6;
+    // 1 key of 128 7.5 / 7.7, and of 64 with values of 128 6.8 / 7.4 (the only sizes tried that lose more than 0.3 us).
+    if constexpr (LINES)
     {
-        if (k_vec && dim % 64 == 0 && vdim % 64 == 0 && (uintptr_t) vb % 16 == 0 && v_step % 8 == 0 && k_step < (1 << 27) && v_step < (1 << 27))
+        constexpr bool AHEAD = MAXV == 1 || NW <= 8;                 // registers for the values next to the keys; else the values follow the scores and keys come four at a time
+        constexpr int KR = AHEAD ? 8 : 4;
+        const int kg = lane >> 3, kp = lane & 7;
+        float va[MAXV][8];
+        #pragma unroll
+        for (int i = 0; i < MAXV; ++i)
+            #pragma unroll
+            for (int e = 0; e < 8; ++e) va[i][e] = 0.f;
+        union piece { uint4 v; T e[8]; };
+        // the eight rows from j on (past the end: the last one): where they lie in a line, a scalar base and a 32-bit offset per lane -- 16 waves leave 128 registers each
+        auto rows = [&] (const T* base, int64_t step, int j, int c) __attribute__((always_inline)) -> uint4
         {
-            constexpr bool AHEAD = MAXV == 1 || NW <= 8;                 // registers for the values next to the keys; else the values follow the scores and keys come four at a time
-            constexpr int KR = AHEAD ? 8 : 4;
-            const int kg = lane >> 3, kp = lane & 7;
-            float va[MAXV][8];
-            #pragma unroll
-            for (int i = 0; i < MAXV; ++i)
-                #pragma unroll
-                for (int e = 0; e < 8; ++e) va[i][e] = 0.f;
-            union piece { uint4 v; T e[8]; };
-            // the eight rows from j on (past the end: the last one): where they lie in a line, a scalar base and a 32-bit offset per lane -- 16 waves leave 128 registers each
-            auto rows = [&] (const T* base, int64_t step, int j, int c) __attribute__((always_inline)) -> uint4
+            const int first = min(j, count - 1);
+            if constexpr (RowMap::linear) return *(const uint4*) (base + first * step + c + (min(kg, count - 1 - first) * (int) step + 8 * kp));
+            else return *(const uint4*) (base + map(min(j + kg, count - 1)) * step + c + 8 * kp);
+        };
+        // chunks of 8 .. 64 keys: a row too short for 64 to every wave is shared by more of them, each with a shorter chain of loads (64 keys of 128 dimensions: 12.4 us in one chunk, 8.6)
+        const int chunk = min(64, (count + 8 * NW - 1) / (8 * NW) * 8);
+        for (int j0 = w * chunk; j0 < count; j0 += chunk * NW)
+        {
+            const int here = min(chunk, count - j0);                // keys of this chunk: eight rows at a time are skipped behind the last
+            float d[8];
+            piece tv[8];
+            auto values = [&] (int c)
             {
-                const int first = min(j, count - 1);
-                if constexpr (RowMap::linear) return *(const uint4*) (base + first * step + c + (min(kg, count - 1 - first) * (int) step + 8 * kp));
-                else return *(const uint4*) (base + map(min(j + kg, count - 1)) * step + c + 8 * kp);
+                #pragma unroll
+                for (int i = 0; i < 8; ++i) { if (8 * i >= here) break; tv[i].v = rows(vb, v_step, j0 + 8 * i, c); }
             };
-            for (int j0 = w * 64; j0 < count; j0 += 64 * NW)
+            #pragma unroll
+            for (int i = 0; i < 8; ++i) d[i] = 0.f;
+            for (int c = 0; c < dim; c += 64)
             {
-                float d[8];
-                piece tv[8];
-                auto values = [&] (int c)
-                {
-                    #pragma unroll
-                    for (int i = 0; i < 8; ++i) tv[i].v = rows(vb, v_step, j0 + 8 * i, c);
-                };
+                float qv[8];
                 #pragma unroll
-                for (int i = 0; i < 8; ++i) d[i] = 0.f;
-                for (int c = 0; c < dim; c += 64)
+                for (int e = 0; e < 8; ++e) qv[e] = qs[c + 8 * kp + e];
+                #pragma unroll
+                for (int i0 = 0; i0 < 8; i0 += KR)
                 {
-                    float qv[8];
+                    piece tk[KR];
                     #pragma unroll
-                    for (int e = 0; e < 8; ++e) qv[e] = qs[c + 8 * kp + e];
+                    for (int i = 0; i < KR; ++i) { if (8 * (i0 + i) >= here) break; tk[i].v = rows(kb, k_step, j0 + 8 * (i0 + i), c); }
+                    if (AHEAD && c == 0 && i0 + KR == 8) values(0);
                     #pragma unroll
-                    for (int i0 = 0; i0 < 8; i0 += KR)
+                    for (int i = 0; i < KR; ++i)
                     {
-                        piece tk[KR];
+                        if (8 * (i0 + i) >= here) break;
                         #pragma unroll
-                        for (int i = 0; i < KR; ++i) tk[i].v = rows(kb, k_step, j0 + 8 * (i0 + i), c);
-                        if (AHEAD && c == 0 && i0 + KR == 8) values(0);
-                        #pragma unroll
-                        for (int i = 0; i < KR; ++i)
-                            #pragma unroll
-                            for (int e = 0; e < 8; ++e) d[i0 + i] += qv[e] * to_f(tk[i].e[e]);
+                        for (int e = 0; e < 8; ++e) d[i0 + i] += qv[e] * to_f(tk[i].e[e]);
                     }
                 }
-                #pragma unroll
-                for (int i = 0; i < 8; ++i) d[i] = row8_sum(d[i]);
-                if (kp == 0)
-                {
-                    #pragma unroll
-                    for (int i = 0; i < 8; ++i) pw[8 * i + kg] = d[i];
-                }
-                __builtin_amdgcn_wave_barrier();
-                float s = pw[lane] * scale;
-                if (softcap > 0.f) s = softcap * tanhf(s / softcap);
-                if (j0 + lane >= count) s = -INFINITY;
-                const float m_new = fmaxf(m, wave_max(s));
-                const float p = j0 + lane < count ? expf(s - m_new) : 0.f, corr = expf(m - m_new);
-                l = l * corr + wave_sum(p);
-                m = m_new;
-                __builtin_amdgcn_wave_barrier();
-                pw[lane] = p;
-                __builtin_amdgcn_wave_barrier();
-                #pragma unroll
-                for (int i = 0; i < MAXV; ++i)
-                {
-                    if (64 * i >= vdim) continue;
-                    if (i > 0 || !AHEAD) values(64 * i);
-                    #pragma unroll
-                    for (int e = 0; e < 8; ++e) va[i][e] *= corr;
-                    #pragma unroll
-                    for (int r = 0; r < 8; ++r)
-                    {
-                        const bool in = j0 + 8 * r + kg < count;
-                        const float pr = pw[8 * r + kg];
-                        #pragma unroll
-                        for (int e = 0; e < 8; ++e) va[i][e] += in ? pr * to_f(tv[r].e[e]) : 0.f;
-                    }
-                }
-                __builtin_amdgcn_wave_barrier();
             }
-            float* part = mg + w * (2 + MAXV * 64);
-            if (lane == 0) { part[0] = m; part[1] = l; }
+            #pragma unroll
+            for (int i = 0; i < 8; ++i) d[i] = row8_sum(d[i]);
+            if (kp == 0)
+            {
+                #pragma unroll
+                for (int i = 0; i < 8; ++i) pw[8 * i + kg] = d[i];
+            }
+            __builtin_amdgcn_wave_barrier();
+            float s = pw[lane] * scale;
+            if (softcap > 0.f) s = softcap * tanhf(s / softcap);
+            if (lane >= here) s = -INFINITY;
+            const float m_new = fmaxf(m, wave_max(s));
+            const float p = lane < here ? expf(s - m_new) : 0.f, corr = expf(m - m_new);
+            l = l * corr + wave_sum(p);
+            m = m_new;
+            __builtin_amdgcn_wave_barrier();
+            pw[lane] = p;
+            __builtin_amdgcn_wave_barrier();
+            #pragma unroll
+            for (int i = 0; i < MAXV; ++i)
+            {
+                if (64 * i >= vdim) continue;
+                if (i > 0 || !AHEAD) values(64 * i);
+                #pragma unroll
+                for (int e = 0; e < 8; ++e) va[i][e] *= corr;
+                #pragma unroll
+                for (int r = 0; r < 8; ++r)
+                {
+                    if (8 * r >= here) break;
+                    const bool in = 8 * r + kg < here;
+                    const float pr = pw[8 * r + kg];
+                    #pragma unroll
+                    for (int e = 0; e < 8; ++e) va[i][e] += in ? pr * to_f(tv[r].e[e]) : 0.f;
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
+        float* part = mg + w * (2 + MAXV * 64);
+        if (lane == 0) { part[0] = m; part[1] = l; }
+        if (w * chunk < count)
+        {
             #pragma unroll
             for (int i = 0; i < MAXV; ++i)
                 #pragma unroll
-                for (int e = 0; e < 8; ++e)
-                {
-                    float a = va[i][e];
-                    a += __shfl_xor(a, 8, 64); a += __shfl_xor(a, 16, 64); a += __shfl_xor(a, 32, 64);
-                    if (kg == 0) part[2 + 64 * i + 8 * kp + e] = a;
-                }
-            attn_row_merge<T, MAXV, TO, NW>(out, vdim, gate, mg, gate_row);
-            return;
+                for (int e = 0; e < 8; ++e) va[i][e] = sum_of_8th_lanes(va[i][e]);
         }
+        if (kg == 0)
+        {
+            #pragma unroll
+            for (int i = 0; i < MAXV; ++i)
+                #pragma unroll
+                for (int e = 0; e < 8; ++e) part[2 + 64 * i + 8 * kp + e] = va[i][e];
+        }
+        attn_row_merge<T, MAXV, TO, NW>(out, vdim, gate, mg, gate_row);
+        return;
     }
     for (int j0 = w * 64; j0 < count; j0 += 64 * NW)
     {

@@ -58,6 +58,16 @@ __device__ __forceinline__ float row8_sum(float v)
     return v;
 }
 
+// sum over the lanes of equal lane % 8, every one of them gets it: lane ^ 8 by half a turn of a row, ^ 16 and ^ 32 by swaps of rows between two copies
+__device__ __forceinline__ float sum_of_8th_lanes(float v)
+{
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, true));
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+
 // sum over a workgroup of NW waves; every thread gets the result.  `red` holds NW floats; two barriers.
 template <int NW>
 __device__ __forceinline__ float block_sum(float v, float* red)

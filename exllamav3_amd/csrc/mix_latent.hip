@@ -184,7 +184,7 @@ __global__ __launch_bounds__(256) void rotate_heads_kernel(T* __restrict__ q, in
 }
 
 // PAGED: the cached rows of a sequence lie in pages of `page` rows listed by its row of `table`; otherwise in the slot's ring of `window` rows
-template <typename T, int MAXV, bool PAGED>
+template <typename T, int MAXV, bool PAGED, bool LINES>
 __global__ __launch_bounds__(64 * AT_WAVES) void latent_decode_kernel(T* __restrict__ o_lat, int64_t o_row, int64_t o_head, const T* __restrict__ q_lat, int64_t ql_row,
                                                                       int64_t ql_head, const T* __restrict__ q, int64_t q_ld, const T* __restrict__ ring,
                                                                       const float* __restrict__ sink, const int32_t* __restrict__ slots,
@@ -196,14 +196,14 @@ __global__ __launch_bounds__(64 * AT_WAVES) void latent_decode_kernel(T* __restr
     const int row = rank + rot_dim;
     if constexpr (PAGED)
     {
-        attn_row<T, MAXV, T, AT_WAVES, row_paged>(o_lat + (int64_t) n * o_row + (int64_t) h * o_head, q_lat + (int64_t) n * ql_row + (int64_t) h * ql_head,
+        attn_row<T, MAXV, LINES, T, AT_WAVES, row_paged>(o_lat + (int64_t) n * o_row + (int64_t) h * o_head, q_lat + (int64_t) n * ql_row + (int64_t) h * ql_head,
                       q + (int64_t) n * q_ld + (int64_t) h * (dim + rot_dim) + dim, rank, ring, row, ring, row, len_after[n], row, rank, scale,
                       sink != nullptr, sink ? sink[h] : 0.f, 1.0f, rows_are_16_byte(ring, (int64_t) row, row), smem, 0.f, row_paged{table + (int64_t) slots[n] * table_ld, page});
         return;
     }
     const int count = min(len_after[n], window);
     const T* kb = ring + (int64_t) slots[n] * window * row;
-    attn_row<T, MAXV>(o_lat + (int64_t) n * o_row + (int64_t) h * o_head, q_lat + (int64_t) n * ql_row + (int64_t) h * ql_head,
+    attn_row<T, MAXV, LINES>(o_lat + (int64_t) n * o_row + (int64_t) h * o_head, q_lat + (int64_t) n * ql_row + (int64_t) h * ql_head,
                       q + (int64_t) n * q_ld + (int64_t) h * (dim + rot_dim) + dim, rank, kb, row, kb, row, count, row, rank, scale,
                       sink != nullptr, sink ? sink[h] : 0.f, 1.0f, rows_are_16_byte(kb, (int64_t) row, row), smem);
 }
@@ -271,13 +271,16 @@ extern "C" int exl3_mix_latent_decode(void* o_lat, int64_t o_row, int64_t o_head
     const int mv = (rank + 63) / 64;
     const int mvt = mv == 1 ? 1 : (mv == 2 ? 2 : (mv <= 4 ? 4 : (mv <= 8 ? 8 : 16)));
     const size_t sm = (size_t) (rank + rot_dim + AT_WAVES * 64 + AT_WAVES * (2 + mvt * 64)) * sizeof(float);
-    #define LD_LAUNCH_P(MV, PG) hipLaunchKernelGGL((latent_decode_kernel<T, MV, PG>), dim3(n, heads), dim3(64 * AT_WAVES), sm, (hipStream_t) stream, (T*) o_lat, o_row, o_head, \
+    const bool lines = rows_of_lines(ring, rank + rot_dim, ring, rank + rot_dim, rank + rot_dim, rank);
+    #define LD_LAUNCH_P(MV, PG, LI) hipLaunchKernelGGL((latent_decode_kernel<T, MV, PG, LI>), dim3(n, heads), dim3(64 * AT_WAVES), sm, (hipStream_t) stream, (T*) o_lat, o_row, o_head, \
                                              (const T*) q_lat, ql_row, ql_head, (const T*) q, q_ld, (const T*) ring, sink, slots, len_after, table, table_ld, page, \
                                              dim, rot_dim, rank, scale, window)
-    #define LD_LAUNCH(MV) do { if (table) LD_LAUNCH_P(MV, true); else LD_LAUNCH_P(MV, false); } while (0)
+    #define LD_LAUNCH_F(MV, LI) do { if (table) LD_LAUNCH_P(MV, true, LI); else LD_LAUNCH_P(MV, false, LI); } while (0)
+    #define LD_LAUNCH(MV) do { if (MV <= 4 && sizeof(T) == 2 && lines) LD_LAUNCH_F(MV, (MV <= 4 && sizeof(T) == 2)); else LD_LAUNCH_F(MV, false); } while (0)
     MIX_DISPATCH_T(dtype,
         if (mv == 1) LD_LAUNCH(1); else if (mv == 2) LD_LAUNCH(2); else if (mv <= 4) LD_LAUNCH(4); else if (mv <= 8) LD_LAUNCH(8); else LD_LAUNCH(16));
     #undef LD_LAUNCH
+    #undef LD_LAUNCH_F
     #undef LD_LAUNCH_P
     return mix_check_launch("mix_latent_decode");
 }

@@ -94,3 +94,26 @@ def test_decode_attention_rows_of_whole_lines(dim, vdim, H, G, window):
         e = torch.exp(torch.cat([s, sink.double().view(H, 1)], dim=1) - torch.maximum(s.amax(1), sink.double()).view(H, 1))
         want = torch.einsum("hc,chv->hv", e[:, :c] / e.sum(1, keepdim=True), v)
         assert _rel(out[b].view(H, vdim), want) < 2.5e-3, l
+
+
+@pytest.mark.parametrize("dim,vdim,H,G,window", [(64, 64, 4, 2, 1100), (128, 128, 2, 1, 1100), (64, 256, 2, 2, 1100), (64, 64, 40, 8, 300), (128, 192, 40, 8, 300)])
+def test_decode_attention_rows_where_the_chunks_change(dim, vdim, H, G, window):
+    """Rows are cut into chunks of 8 to 64 keys by their length: the lengths where a chunk grows, over 16 waves (few rows of a long window) and over 4.
+    Bound: the output's rounding to 8 bits, 2^-9 / sqrt(3), over sums of exact products in float32."""
+    from exllamav3_amd import mix_ops
+    gen = torch.Generator(device=DEV).manual_seed(dim + vdim + H)
+    rnd = lambda *s: torch.randn(*s, device=DEV, generator=gen).bfloat16()
+    waves = 16 if H < 10 else 4
+    lens = [l for g in (1, 2, 7) for l in (8 * waves * g - 1, 8 * waves * g, 8 * waves * g + 1) if l <= window]
+    n = len(lens)
+    q, rk, rv = rnd(n, H * dim), rnd(n, window, G, dim), rnd(n, window, G, vdim)
+    for b, l in enumerate(lens):
+        rk[b, l - 1] *= 4                                                 # the last key of a row counts: a lost one shows
+        rk[b, l:], rv[b, l:] = float("nan"), float("nan")
+    mk = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    out = torch.empty((n, H * vdim), dtype=torch.bfloat16, device=DEV)
+    mix_ops.attn_decode(out, q, rk, rv, None, None, mk(list(range(n))), mk(lens), H, dim ** -0.5)
+    for b, l in enumerate(lens):
+        k, v = (t[b, :l].double().repeat_interleave(H // G, dim=1) for t in (rk, rv))
+        p = torch.softmax(torch.einsum("hd,chd->hc", q[b].double().view(H, dim), k) * dim ** -0.5, dim=1)
+        assert _rel(out[b].view(H, vdim), torch.einsum("hc,chv->hv", p, v)) < 2.5e-3, l
