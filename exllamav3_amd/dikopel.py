@@ -26,7 +26,7 @@ import os
 import torch
 from . import mix_ops
 from .loader import SafetensorsCollection
-from .modules import GatedDeltaRule, GatedMLP, MatrixLSTM, ParallelBlock, ParallelMixer, SigmoidAttention, SparseExperts, _f32, _w, linear
+from .modules import GatedDeltaRule, GatedMLP, MatrixLSTM, ParallelBlock, ParallelMixer, SigmoidAttention, SparseExperts, _f32, _w, head_logits
 from .state_cache import SlotStateCache, StepBatch
 
 # a group of experts is scored by the sum of this many of its largest choice scores; the position vector's base
@@ -139,4 +139,4 @@ class DikopelModel:
             return None
         hw = torch.empty((sb.want_rows.numel(), w), dtype=self.dtype, device=self.device)
         mix_ops.layer_norm_rows(hw, x, sb.want_rows, self.final_w, self.final_b, self.cfg.eps)
-        return linear(hw, self.head).float()
+        return head_logits(hw, self.head)

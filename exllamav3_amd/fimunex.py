@@ -22,7 +22,7 @@ import os
 import torch
 from . import mix_ops
 from .loader import SafetensorsCollection
-from .modules import CanonBlock, DifferentialAttention, SparseExperts, _f32, _w, linear
+from .modules import CanonBlock, DifferentialAttention, SparseExperts, _f32, _w, head_logits
 from .state_cache import SlotStateCache, StepBatch
 
 
@@ -128,7 +128,7 @@ class FimunexModel:
             return None
         hw = torch.empty((sb.want_rows.numel(), w), dtype=self.dtype, device=self.device)
         mix_ops.rms_norm_rows(hw, x, sb.want_rows, self.final_norm, self.cfg.eps)
-        logits = linear(hw, self.head).float()
+        logits = head_logits(hw, self.head)
         if self.cfg.logit_softcap:
             mix_ops.softcap(logits, self.cfg.logit_softcap)
         return logits

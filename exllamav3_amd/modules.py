@@ -77,6 +77,14 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None) -
     return F.linear(x, w, bias)
 
 
+def head_logits(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """The vocabulary head in float32.  One or two rows of at least 4096 over a large head stream it through the library's own kernel, everything else is a vendor product
+    (us, own kernel / vendor: 4096 x 128256 of 1 row 168 / 188, of 6 199 / 187, of 16 234 / 186; 6144 x 64000 of 2 rows 140 / 179; 8192 x 8192 of 1 row 23.7 / 22.7;
+    3072 x 64000 of 2 rows 77 / 72; 1024 x 128256 of 1 row 53 / 44)."""
+    own = 0 < x.shape[0] <= 2 and x.shape[1] >= 4096 and w.numel() > 1 << 26
+    return (linear(x, w) if own else F.linear(x, w)).float()
+
+
 class FusedInput:
     """Linears that read the same input, stacked into one weight: one matrix product instead of several, and every consumer kernel takes its
     column block in place (row stride = total width).  Parts without a bias get zeros in the fused bias (adding zero is exact)."""

@@ -18,7 +18,7 @@ import os
 import torch
 from . import mix_ops
 from .loader import SafetensorsCollection
-from .modules import GatedLinearAttention, GatedResidualBlock, PolyNormMLP, SlidingSinkAttention, SparseExperts, _f32, _w, linear
+from .modules import GatedLinearAttention, GatedResidualBlock, PolyNormMLP, SlidingSinkAttention, SparseExperts, _f32, _w, head_logits
 from .state_cache import SlotStateCache, StepBatch
 
 
@@ -100,4 +100,4 @@ class VofanexModel:
             return None
         hw = torch.empty((sb.want_rows.numel(), w), dtype=self.dtype, device=self.device)
         mix_ops.rms_norm_rows(hw, x, sb.want_rows, self.final_norm, self.cfg.eps)
-        return linear(hw, self.head).float()
+        return head_logits(hw, self.head)

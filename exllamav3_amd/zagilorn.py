@@ -22,7 +22,7 @@ import torch
 import torch.nn.functional as F
 from . import mix_ops
 from .loader import SafetensorsCollection
-from .modules import ActMLP, DynTanh, GatedMLP, LatentAttention, NextInput, PreNormBlock, SparseExperts, TokenSide, update_residual, _w, linear
+from .modules import ActMLP, DynTanh, GatedMLP, LatentAttention, NextInput, PreNormBlock, SparseExperts, TokenSide, update_residual, _w, head_logits, linear
 from .state_cache import SlotStateCache, StepBatch
 
 MIXER_TYPES = {"latent_attention": dict(sink=True, gate=True), "latent_attention_2": dict(sink=False, gate=False)}
@@ -155,5 +155,5 @@ class ZagilornModel:
             return None
         hw = torch.empty((sb.want_rows.numel(), w), dtype=self.dtype, device=self.device)
         mix_ops.dyn_tanh_rows(hw, x, sb.want_rows, self.final_norm.alpha, self.final_norm.w, self.final_norm.b)
-        logits = linear(hw, self.head).float()
+        logits = head_logits(hw, self.head)
         return logits * self.cfg.logit_scale if self.cfg.logit_scale != 1.0 else logits
