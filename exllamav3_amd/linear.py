@@ -26,6 +26,9 @@ FUSED_RECONSTRUCT_MIN_ROWS = AUTO_RECONSTRUCT_THRESHOLD + 1
 
 # ext.dgemm ends below this many rows: from 1024 on prompt chunks may have their weights rebuilt ahead on a second stream (ReconstructAhead) and give the same bits either way.  Below, sizes, bits per
 # weight and codebook decide (ext.dgemm_pays): 14336 x 4096 at 1000 rows 131 us against 148 through rebuilt weights (4 bits), 4096 x 14336 at 512 rows 77 / 83, at 560 rows 94 / 88.
+# Error: this route rounds the rotated rows to fp16 and multiplies by the exact weights, the other multiplies the rows as they come by a W^T rounded to fp16 on both sides of its scales.  Relative
+# to 64 bits (4096 -> 1024, 14336 -> 512, 2048 -> 8192 at 150, 400 and 1000 rows, 2 to 8 bits, three codebooks, inputs with and without outlier columns): 2.0 - 2.1e-4 here and 2.8 - 3.0e-4 there
+# before the output's own rounding, 2.9 - 3.0e-4 and 3.5 - 3.6e-4 in fp16, smaller here in every call.
 DGEMM_MAX_ROWS = 1023
 
 #: the fused prefill GEMMs reconstruct their matrices with ONE launch (ext.reconstruct_had_multi_t); EXL3_HIP_RECON_MULTI=0: one launch per matrix

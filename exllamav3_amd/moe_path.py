@@ -37,7 +37,9 @@ class SyntheticEXL3MoE:
     grouped_prefill = True
 
     #: forward_prefill: mean rows per expert up to which the grouped products decode the packed weights themselves.  Mixtral's block (4096 / 14336, 8 experts, top 2, 4 bpw), us for
-    #: reconstructed weights / packed ones: 130 tokens 1763 / 380, 600: 1751 / 626, 1100: 2056 / 1079, 2000: 2342 / 1973, 2500: 2772 / 2461, 3000: 2793 / 3045, 4096: 3596 / 4039
+    #: reconstructed weights / packed ones: 130 tokens 1808 / 391, 800: 1824 / 835, 1280: 2097 / 1273, 2160: 2720 / 2216, 2560: 2799 / 2506, 3040: 2930 / 3071.  The line holds for other blocks too
+    #: (4096 / 1536, 2048 / 768, 2048 / 1024 and 5120 / 8192 of 64, 128, 64 and 16 experts; 2 to 8 bits, three codebooks): packed over reconstructed 0.77 - 0.94 at 540 rows per expert, 0.86 - 1.02 at
+    #: 640 (1.02: 8 bits, codebook 0, 5120 / 8192), 0.94 - 1.11 at 760
     DGEMM_ROWS = 640
 
     # k-slices of the fx block's gate|up / down launches (0: the dispatcher / the rule in forward_fx); EXL3_HIP_MOE_FX_SPLIT="g,d" overrides (tuning)
