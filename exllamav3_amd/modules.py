@@ -78,10 +78,13 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None) -
 
 
 def head_logits(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """The vocabulary head in float32.  One or two rows of at least 4096 over a large head stream it through the library's own kernel, everything else is a vendor product
-    (us, own kernel / vendor: 4096 x 128256 of 1 row 168 / 188, of 6 199 / 187, of 16 234 / 186; 6144 x 64000 of 2 rows 140 / 179; 8192 x 8192 of 1 row 23.7 / 22.7;
-    3072 x 64000 of 2 rows 77 / 72; 1024 x 128256 of 1 row 53 / 44)."""
-    own = 0 < x.shape[0] <= 2 and x.shape[1] >= 4096 and w.numel() > 1 << 26
+    """The vocabulary head in float32: the library's own kernel for few rows where it is the faster product, else a vendor product.  Bound by the weights' way from memory, which a decode step
+    finds cold.  Measured with the weights rotated through 1.3 GB, 8 widths x 15 vocabularies x 1 .. 16 rows (us, own / vendor): the vendor's kernels lose a fifth where a row is a multiple of 4 KB
+    (2048 x 32000 of 1, 8, 16 rows 30 / 36, 32 / 34, 36 / 35; 4096 x 64000 of 1, 4, 16 rows 90 / 120, 100 / 117, 123 / 120; 8192 x 128256 of 2, 4 rows 359 / 362, 371 / 356), the own one slows down
+    with rows x width; elsewhere the vendor is ahead (1024 x 128256 of 1 row 65 / 57; 2560 x 64000 70 / 64) but on small heads (1024 x 8192 8 / 10, 3072 x 4096 9 / 14).  At worst 7 % behind the
+    vendor's, 2048 x 50257 of 8 rows."""
+    n, width, vocab = x.shape[0], x.shape[1], w.shape[0]
+    own = (width % 2048 == 0 and n * width <= 16384) or (vocab <= 8192 and (n <= 4 or width <= 3072))
     return (linear(x, w) if own else F.linear(x, w)).float()
 
 
