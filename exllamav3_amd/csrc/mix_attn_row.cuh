@@ -80,7 +80,10 @@ __device__ __forceinline__ void attn_row(TO* __restrict__ out, const T* __restri
     float* qs = smem;                                   // [dim]
     float* ps = qs + dim;                               // [NW][64]
     float* mg = ps + NW * 64;                     // [NW][2 + MAXV * 64]: m, l, accumulators
-    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // the wave's index as a scalar helps the forms below whose loads leave registers (float32 of up to 256 values: 0.91 of the time) and costs one key per lane in bfloat16 2 to 10 %, in float32 over
+    // 256 values up to 80 % (8 heads of 320, 1 key: 8.0 us, 14.6)
+    constexpr bool SCALAR_WAVE = LINES || (sizeof(T) == 4 && MAXV <= 4);
+    const int lane = threadIdx.x & 63, w = SCALAR_WAVE ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : (int) (threadIdx.x >> 6);
     for (int i = threadIdx.x; i < dim; i += 64 * NW) qs[i] = to_f(i < dim1 ? q[i] : q2[i - dim1]);      // the query may come in two parts
     __syncthreads();
     const bool seeded = has_sink && w == 0;
