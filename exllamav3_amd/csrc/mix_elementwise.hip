@@ -29,8 +29,8 @@ template <typename T> __host__ __device__ constexpr int wide_n() { return 16 / (
 #define ROW_HELD 4
 
 // h = x inv w for the row whose first pieces are in `held`; the others come from x, which the same thread wrote or read
-template <typename T, int V, int NT = ROW_THREADS>
-__device__ __forceinline__ void row_norm_write(T* __restrict__ hr, const float* xr, const float* __restrict__ w, const float (&held)[ROW_HELD][V], float inv, int width)
+template <typename T, int V, int NT = ROW_THREADS, int HELD = ROW_HELD>
+__device__ __forceinline__ void row_norm_write(T* __restrict__ hr, const float* xr, const float* __restrict__ w, const float (&held)[HELD][V], float inv, int width)
 {
     auto write = [&] (int i, const float (&v)[V]) __attribute__((always_inline))
     {
@@ -41,8 +41,8 @@ __device__ __forceinline__ void row_norm_write(T* __restrict__ hr, const float* 
         store_n<T, V>(hr + i, wv);
     };
     #pragma unroll
-    for (int u = 0; u < ROW_HELD; ++u) { const int i = (u * NT + threadIdx.x) * V; if (i < width) write(i, held[u]); }
-    for (int i = (ROW_HELD * NT + threadIdx.x) * V; i < width; i += NT * V) { float t[V]; load_n<float, V>(xr + i, t); write(i, t); }
+    for (int u = 0; u < HELD; ++u) { const int i = (u * NT + threadIdx.x) * V; if (i < width) write(i, held[u]); }
+    for (int i = (HELD * NT + threadIdx.x) * V; i < width; i += NT * V) { float t[V]; load_n<float, V>(xr + i, t); write(i, t); }
 }
 
 template <typename T, int V>
@@ -105,7 +105,7 @@ __global__ __launch_bounds__(ROW_THREADS) void rms_norm_rows_kernel(T* __restric
     row_norm_write<T, V>(h + (int64_t) n * width, xr, w, held, inv, width);
 }
 
-template <typename T, int V, int NW>
+template <typename T, int V, int NW, int HELD>
 __global__ __launch_bounds__(64 * NW) void gated_residual_kernel(float* __restrict__ x, const T* __restrict__ y, int64_t y_ld, const T* __restrict__ r,
                                                                      int64_t r_ld, const float* __restrict__ norm_w, T* __restrict__ h, float eps, int width)
 {
@@ -115,7 +115,7 @@ __global__ __launch_bounds__(64 * NW) void gated_residual_kernel(float* __restri
     float* xr = x + (int64_t) n * width;
     const T* yr = y + (int64_t) n * y_ld;
     const T* rr = r + (int64_t) n * r_ld;
-    float held[ROW_HELD][V], yv[ROW_HELD][V], rv[ROW_HELD][V];
+    float held[HELD][V], yv[HELD][V], rv[HELD][V];
     float ss = 0.f;
     auto form = [&] (int i, float (&v)[V], const float (&a)[V], const float (&g)[V]) __attribute__((always_inline))
     {
@@ -124,14 +124,14 @@ __global__ __launch_bounds__(64 * NW) void gated_residual_kernel(float* __restri
         store_n<float, V>(xr + i, v);
     };
     #pragma unroll
-    for (int u = 0; u < ROW_HELD; ++u)
+    for (int u = 0; u < HELD; ++u)
     {
         const int i = (u * NT + threadIdx.x) * V;
         if (i < width) { load_n<float, V>(xr + i, held[u]); load_n<T, V>(yr + i, yv[u]); load_n<T, V>(rr + i, rv[u]); }
     }
     #pragma unroll
-    for (int u = 0; u < ROW_HELD; ++u) { const int i = (u * NT + threadIdx.x) * V; if (i < width) form(i, held[u], yv[u], rv[u]); }
-    for (int i = (ROW_HELD * NT + threadIdx.x) * V; i < width; i += NT * V)
+    for (int u = 0; u < HELD; ++u) { const int i = (u * NT + threadIdx.x) * V; if (i < width) form(i, held[u], yv[u], rv[u]); }
+    for (int i = (HELD * NT + threadIdx.x) * V; i < width; i += NT * V)
     {
         float v[V], a[V], g[V];
         load_n<float, V>(xr + i, v); load_n<T, V>(yr + i, a); load_n<T, V>(rr + i, g);
@@ -140,7 +140,7 @@ __global__ __launch_bounds__(64 * NW) void gated_residual_kernel(float* __restri
     if (!norm_w) return;
     ss = block_sum<NW>(ss, red);
     const float inv = 1.0f / sqrtf(ss / (float) width + eps);
-    row_norm_write<T, V, NT>(h + (int64_t) n * width, xr, norm_w, held, inv, width);
+    row_norm_write<T, V, NT, HELD>(h + (int64_t) n * width, xr, norm_w, held, inv, width);
 }
 
 template <typename T, int V, int NW>
@@ -223,7 +223,8 @@ extern "C" int exl3_mix_embed(float* x, void* h, const void* table, const int32_
     MIX_CHECK(x && table && tokens && n >= 0 && width > 0 && vocab > 0 && (!norm_w || h), "mix_embed: bad arguments");
     if (n == 0) return EXL3_MIX_OK;
     #define EMBED(VV) hipLaunchKernelGGL((embed_kernel<T, VV>), dim3(n), dim3(ROW_THREADS), 0, (hipStream_t) stream, x, (T*) h, (const T*) table, tokens, scale, norm_w, eps, width, vocab)
-    MIX_DISPATCH_T(dtype, if (row_wide<T>(width, width) && aligned16(x, h, table, norm_w)) EMBED(wide_n<T>()); else EMBED(1));
+    // (up to 256 wide 16 bytes a lane leave most lanes idle: 128 wide, 4096 rows 5.1 us, 4.5 with one element)
+    MIX_DISPATCH_T(dtype, if (width > 256 && row_wide<T>(width, width) && aligned16(x, h, table, norm_w)) EMBED(wide_n<T>()); else EMBED(1));
     #undef EMBED
     return mix_check_launch("mix_embed");
 }
@@ -243,9 +244,14 @@ extern "C" int exl3_mix_gated_residual(float* x, const void* y, int64_t y_ld, co
 {
     MIX_CHECK(x && y && r && n >= 0 && width > 0 && y_ld >= width && r_ld >= width && (!norm_w || h), "mix_gated_residual: bad arguments");
     if (n == 0) return EXL3_MIX_OK;
-    // (1000 wide, 4096 rows of bfloat16: 14.4 us with four waves, 11.6 with the two that the row keeps busy)
-    #define GATED(VV, NW) hipLaunchKernelGGL((gated_residual_kernel<T, VV, NW>), dim3(n), dim3(64 * NW), 0, (hipStream_t) stream, x, (const T*) y, y_ld, (const T*) r, r_ld, norm_w, (T*) h, eps, width)
-    MIX_DISPATCH_T(dtype, if (row_wide<T>(width, y_ld) && row_wide<T>(width, r_ld) && aligned16(x, y, r, norm_w) && aligned16(h, nullptr, nullptr, nullptr)) { if (width <= 128 * wide_n<T>()) GATED(wide_n<T>(), 2); else GATED(wide_n<T>(), 4); } else GATED(1, 4));
+    // 1000 wide, 4096 rows of bfloat16: 14.4 us with four waves, 11.6 with the two that the row keeps busy.  Short rows leave most lanes idle at 16 bytes each (8 rows, us with
+    // one element a lane: 96 wide 3.0 / 2.3, 512 wide 2.8 / 2.6; 4096 rows of 512 10.1 / 11.2).  Single elements: one piece held -- four make long rows wait for more than they hide (2050 wide, 4096 rows 33.6 us with four, 30.7 with one) -- and, while the rows are too few to fill the
+    // chip, eight waves (2050 wide, us of four / eight: 1 row 4.7 / 3.4, 1024 rows 12.2 / 10.2, 4096 rows 30.7 / 35.6).
+    #define GATED(VV, NW, H) hipLaunchKernelGGL((gated_residual_kernel<T, VV, NW, H>), dim3(n), dim3(64 * NW), 0, (hipStream_t) stream, x, (const T*) y, y_ld, (const T*) r, r_ld, norm_w, (T*) h, eps, width)
+    MIX_DISPATCH_T(dtype, constexpr int V = wide_n<T>();
+                          const bool wide = width > (n <= 1024 ? 512 : 256) && row_wide<T>(width, y_ld) && row_wide<T>(width, r_ld) && aligned16(x, y, r, norm_w) && aligned16(h, nullptr, nullptr, nullptr);
+                          if (wide && width <= 128 * V) GATED(V, 2, ROW_HELD); else if (wide) GATED(V, 4, ROW_HELD);
+                          else if (width > 512 && n <= 1024) GATED(1, 8, 1); else GATED(1, 4, 1));
     #undef GATED
     return mix_check_launch("mix_gated_residual");
 }
@@ -254,9 +260,10 @@ extern "C" int exl3_mix_polynorm(void* out, const void* z, int64_t z_ld, const f
 {
     MIX_CHECK(out && z && coef && n >= 0 && ff > 0 && z_ld >= ff, "mix_polynorm: bad arguments");
     if (n == 0) return EXL3_MIX_OK;
-    // waves that a row keeps busy (bfloat16, 4096 rows, us with 8 waves / here: 1000 wide 14.9 / 7.3, 2048 wide 17.4 / 11.6; single elements, 2050 wide 17.6 / 14.7)
+    // waves that a row keeps busy (bfloat16, 4096 rows, us with 8 waves / here: 1000 wide 14.9 / 7.3, 2048 wide 17.4 / 11.6; single elements, 2050 wide 17.6 / 14.7; 96 wide, 8 rows 2.6
+    // with 16 bytes a lane, 2.4 with one element, 4096 rows 5.0 / 6.5)
     #define POLY(VV, NW) hipLaunchKernelGGL((polynorm_kernel<T, VV, NW>), dim3(n), dim3(64 * NW), 0, (hipStream_t) stream, (T*) out, (const T*) z, z_ld, coef, eps, ff)
-    MIX_DISPATCH_T(dtype, constexpr int V = wide_n<T>(); if (!row_wide<T>(ff, z_ld) || !aligned16(out, z, nullptr, nullptr)) POLY(1, 4); else if (ff <= 128 * V) POLY(V, 2);
+    MIX_DISPATCH_T(dtype, constexpr int V = wide_n<T>(); if (!row_wide<T>(ff, z_ld) || !aligned16(out, z, nullptr, nullptr) || (ff <= 256 && n <= 1024)) POLY(1, 4); else if (ff <= 128 * V) POLY(V, 2);
                           else if (ff <= 256 * V) POLY(V, 4); else POLY(V, 8));
     #undef POLY
     return mix_check_launch("mix_polynorm");

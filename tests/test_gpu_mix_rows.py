@@ -50,9 +50,27 @@ def test_norms_and_gates(width, off, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("width,off", [(512, 0), (516, 0), (1000, 0), (1032, 0), (2048, 0), (2050, 0)])
+@pytest.mark.parametrize("width,off", [(256, 0), (264, 0), (512, 0), (513, 0), (516, 0), (1000, 0), (1032, 0), (2048, 0), (2050, 0)])
 def test_norms_and_gates_at_the_widths_where_the_waves_change(width, off, dtype):
     test_norms_and_gates(width, off, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,width,off", [(1024, 513, 1), (1025, 513, 1), (1025, 1026, 1), (1024, 512, 0), (1025, 264, 0), (1025, 256, 0), (1024, 256, 0)])
+def test_gate_and_polynorm_where_the_rows_choose_the_form(n, width, off, dtype):
+    """Gated residual: rows off 16 bytes in eight waves up to 1024 rows and four beyond, short rows in single elements up to 1024 rows; polynomial norm of short rows likewise."""
+    from exllamav3_amd import mix_ops
+    gen = torch.Generator(device=DEV).manual_seed(n + width)
+    x, w = torch.randn((n, width), device=DEV, generator=gen), 1 + 0.1 * torch.randn(width, device=DEV, generator=gen)
+    y, r = _cols(n, width, off, dtype, gen), _cols(n, width, off, dtype, gen)
+    h = torch.empty((n, width), dtype=dtype, device=DEV)
+    coef = torch.tensor([0.5, -0.25, 0.125, 0.3], device=DEV)
+    mix_ops.polynorm(h, y, coef, 1e-5)
+    want = sum(c * p / (p.pow(2).mean(-1, keepdim=True) + 1e-5).sqrt() for c, p in zip(coef.double(), (y.double(), y.double() ** 2, y.double() ** 3))) + coef[3].double()
+    assert _rel(h, want) < TOL[dtype]
+    ref = x.double() + y.double() * torch.sigmoid(r.double())
+    mix_ops.gated_residual(x, y, r, w, h, 1e-5)
+    assert _rel(x, ref) < 1e-6 and _rel(h, ref / (ref.pow(2).mean(-1, keepdim=True) + 1e-5).sqrt() * w.double()) < TOL[dtype]
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
