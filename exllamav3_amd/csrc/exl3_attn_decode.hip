@@ -198,7 +198,10 @@ struct AttnQkvArgs
 // NW = waves per workgroup: 4 (one dependent chain per SIMD: the short contexts, where a wave has one step anyway) or 8 (two chains per SIMD: a step is
 // cache words -> dequantize -> 4 score MFMAs -> softmax -> V tile -> 8 transposed reads + MFMAs, ~0.8 us of one wave's latency; at 16 000 tokens the
 // one-wave-per-SIMD form ran 8 such steps back to back per wave)
-template <int GQ, bool FUSED, bool HD64 = false, int NW = 4>
+// ONE: a split is one step of every wave (split_tokens = 16 NW: short contexts, and batches up to two workgroups per CU).  Such a launch is the latency of its chain, so its form has no second
+// step to request and no accumulators to rescale (a test for the first step inside the loop cost the looped form 30 registers and a quarter of its waves).  Same results.
+// One launch with its merge, us, looped / here: 1 sequence of 528 tokens, 32 heads of 64 8.6 / 7.6; 3 of 1259 9.7 / 8.7; 8 of 1000, 32 heads of 128 12.8 / 11.1.
+template <int GQ, bool FUSED, bool HD64, int NW, bool ONE>
 __global__ __launch_bounds__(64 * NW)
 void attn_decode_wide_kernel(const AttnArgs a, const AttnQkvArgs x)
 {
@@ -248,7 +251,8 @@ void attn_decode_wide_kernel(const AttnArgs a, const AttnQkvArgs x)
         r.ks = (aa.k_scales + base)[off]; r.vs = (aa.v_scales + base)[off];
         return r;
     };
-    StepWords w0 = load_step(a, 0), w1 = load_step(a, 1);      // (four steps in flight measured the same: 22.2 vs 21.1 us per layer at 16 000 tokens -- the step is a dependent chain per wave, not a memory wait)
+    StepWords w0 = load_step(a, 0), w1;
+    if constexpr (!ONE) w1 = load_step(a, 1);      // (four steps in flight measured the same: 22.2 vs 21.1 us per layer at 16 000 tokens -- the step is a dependent chain per wave, not a memory wait)
     if constexpr (FUSED)
     {
         // tasks, one per half-wave: 0 .. GQ - 1 = query head h * GQ + task; GQ = the new token's K row, GQ + 1 = its V row (kv head h; only in the
@@ -399,7 +403,7 @@ void attn_decode_wide_kernel(const AttnArgs a, const AttnQkvArgs x)
     for (int nb = 0; nb < 8; ++nb) oc[nb] = float4_t{ 0.f, 0.f, 0.f, 0.f };
     half_t* vw = vt[wave];
 
-    const int nsteps = (al.split_tokens + 16 * NW - 1) / (16 * NW);
+    const int nsteps = ONE ? 1 : (al.split_tokens + 16 * NW - 1) / (16 * NW);
     uint32_t mk_v = 0x001E001Eu;
     asm volatile("" : "+v"(mk_v));
     for (int st = 0; st < nsteps; ++st)
@@ -409,8 +413,8 @@ void attn_decode_wide_kernel(const AttnArgs a, const AttnQkvArgs x)
         const int tk = min(tb + c, t1 - 1);                     // (this lane's token)
         uint32_t kw[4] = { w0.k.x, w0.k.y, w0.k.z, w0.k.w }, vw4[4] = { w0.v.x, w0.v.y, w0.v.z, w0.v.w };
         half_t ksc = w0.ks, vsc = w0.vs;
-        w0 = w1;
-        if (st + 2 < nsteps) w1 = load_step(al, st + 2);            // (two steps ahead; clamped addresses past the split's end are never used)
+        if constexpr (!ONE) w0 = w1;
+        if (!ONE && st + 2 < nsteps) w1 = load_step(al, st + 2);            // (two steps ahead; clamped addresses past the split's end are never used)
         if constexpr (FUSED)
         {
             // the new token's words come from this workgroup's LDS copy (its cache row is being written by this very launch)
@@ -448,7 +452,12 @@ void attn_decode_wide_kernel(const AttnArgs a, const AttnQkvArgs x)
         // accumulator rescale: 4 cross-lane reads, 36 accumulator reads, 32 multiplies) runs in the first step and almost never again; the merge only needs (reference, sum)
         // to be consistent.  A lane sums the probabilities of its own tokens; the lanes of a head are added once, behind the loop.
         const float mine = fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]));
-        if (__any(mine > m_run + 8.0f))
+        if constexpr (ONE)
+        {
+            m_run = fmaxf(mine, m_run);
+            m_run = fmaxf(m_run, xor_lane(m_run, 16)); m_run = fmaxf(m_run, xor_lane(m_run, 32));
+        }
+        else if (__any(mine > m_run + 8.0f))
         {
             float mx = fmaxf(mine, m_run);
             mx = fmaxf(mx, xor_lane(mx, 16)); mx = fmaxf(mx, xor_lane(mx, 32));
@@ -792,9 +801,11 @@ static int attn_decode_impl(const void* q, void* out, const void* k_cache, const
             const int nw_req = g_attn_wide_waves ? g_attn_wide_waves : nw_env;
             const bool nw8 = nw_req ? nw_req == 8 : st_tok >= 128;
             // (sixteen waves -- four chains per SIMD, a 64 KB merge through LDS -- measured like four: 443 vs 443 vs 457 tok/s with eight at 16 000 tokens; not instantiated)
-            #define AW_LAUNCH(GQv, HD64v) \
-                { if (nw8) { if (xq) attn_decode_wide_kernel<GQv, true, HD64v, 8><<<gridw, 512, 0, st>>>(a, *xq); else attn_decode_wide_kernel<GQv, false, HD64v, 8><<<gridw, 512, 0, st>>>(a, AttnQkvArgs{}); } \
-                  else     { if (xq) attn_decode_wide_kernel<GQv, true, HD64v, 4><<<gridw, 256, 0, st>>>(a, *xq); else attn_decode_wide_kernel<GQv, false, HD64v, 4><<<gridw, 256, 0, st>>>(a, AttnQkvArgs{}); } }
+            const bool one = st_tok <= 16 * (nw8 ? 8 : 4);
+            #define AW_ONE(GQv, HD64v, NWv) \
+                { if (one) { if (xq) attn_decode_wide_kernel<GQv, true, HD64v, NWv, true><<<gridw, 64 * NWv, 0, st>>>(a, *xq); else attn_decode_wide_kernel<GQv, false, HD64v, NWv, true><<<gridw, 64 * NWv, 0, st>>>(a, AttnQkvArgs{}); } \
+                  else     { if (xq) attn_decode_wide_kernel<GQv, true, HD64v, NWv, false><<<gridw, 64 * NWv, 0, st>>>(a, *xq); else attn_decode_wide_kernel<GQv, false, HD64v, NWv, false><<<gridw, 64 * NWv, 0, st>>>(a, AttnQkvArgs{}); } }
+            #define AW_LAUNCH(GQv, HD64v) { if (nw8) AW_ONE(GQv, HD64v, 8) else AW_ONE(GQv, HD64v, 4) }
             if (wide_hd64)
             {
                 switch (gq)
@@ -818,6 +829,7 @@ static int attn_decode_impl(const void* q, void* out, const void* k_cache, const
                 default: AW_LAUNCH(8, false) break;
             }
             #undef AW_LAUNCH
+            #undef AW_ONE
             int rcw = exl3_check_launch("attn_decode_wide");
             if (rcw) return rcw;
             if (split_only) { *nsplit_out = ns; return EXL3_OK; }

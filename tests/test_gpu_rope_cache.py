@@ -209,6 +209,18 @@ def test_attn_decode_qcache(dev, kb, vb, lens, hd, hq, hkv):
     assert np.abs(got - ref).max() / np.sqrt((ref ** 2).mean()) < 1e-2
 
 
+@pytest.mark.parametrize("waves,lens", [(0, [1000] * 8 + [937]), (4, [1000] * 8 + [937]), (8, [200, 65, 64]), (0, [192, 65, 63, 1])])
+@pytest.mark.parametrize("hd,hq,hkv", [(128, 16, 4), (64, 32, 8)])
+def test_attn_decode_splits_of_one_step_and_of_several(dev, waves, lens, hd, hq, hkv):
+    """Splits of one step of every wave (128 tokens in eight waves, 64 in four, 64 in eight of which half have nothing) and, with four waves forced on splits of 128, of two."""
+    from exllamav3_amd import ext
+    try:
+        ext.set_attn_wide_waves(waves)
+        test_attn_decode_qcache(dev, 4, 4, lens, hd, hq, hkv)
+    finally:
+        ext.set_attn_wide_waves(0)
+
+
 @pytest.mark.parametrize("kb,vb,hd,hq,hkv", [(4, 4, 128, 8, 2), (8, 3, 128, 4, 4), (4, 4, 64, 8, 2), (2, 6, 64, 32, 8)])
 @pytest.mark.parametrize("lens,max_len", [([1], 1), ([63, 64], 64), ([300, 1000, 77], 1000), ([2500, 1, 700], 2560)])
 def test_attn_decode_qcache_with_sinks(dev, kb, vb, hd, hq, hkv, lens, max_len):
