@@ -248,7 +248,17 @@ extern "C" int exl3_dgemm_pays(int m, int k, int n, int K, int cb)
     if (rc != EXL3_OK) return rc;
     const double kn = 1e-6 * (double) k * n, tiles = (m + 255) / 256;
     const double here = fmax(16.5, 9.5 + 1.243 * dg_plan(m, k, n, K, cb, cus, INT64_MAX).us);
-    const double there = fmax(30.5, 15.3 + 0.669 * kn + 0.126 * kn * tiles + 0.616e-3 * kn * m + 0.88e-3 * k + 1.365e-6 * (double) k * m);
+    // (30.5: the host's time for that route's launches, which is what small calls one after the other take; behind a queue of other work they take their device time, 1024 x 1024 at 1000 rows 21 us here
+    // and 16 there, 2048 x 2048 29 and 26.  Many rows are such a queue: beyond 768 of them the device's time decides, but for long contractions)
+    const double there = fmax(m > 768 && k < 2 * n ? 0.0 : 30.5, 15.3 + 0.669 * kn + 0.126 * kn * tiles + 0.616e-3 * kn * m + 0.88e-3 * k + 1.365e-6 * (double) k * m);
+    if (n >= 10240 && kn >= 55.0)
+    {
+        // Large matrices of many columns: the plain GEMM's tiles of 256 x 256 run in whole rounds over the chip, which the line above knows nothing of (4096 x 22016, 4 bits, 400 rows: 102 us here, 131
+        // there, 126 by that line; 5120 x 27648, 600 rows 224 / 292 / 225).  Fitted to 420 calls of seven shapes, 6.4 % rms; the factor from 840 calls and 330 of gate and up together: the choice is
+        // 0.3 % slower than the better route on average, 11 % at most (4096 x 28672, 8 bits, codebook 0, 512 rows), where the line above was 1.7 and 2.2 % and 35 % slower.
+        const double rounds = ceil(tiles * ceil(n / 256.0) / cus);
+        return here < 1.06 * (-11.5 + 0.805 * kn + 0.584e-3 * kn * m + 2.68e-3 * k * rounds + 0.191 * kn * tiles) ? 1 : 0;
+    }
     return here < 0.97 * there ? 1 : 0;
 }
 

@@ -204,7 +204,8 @@ def test_a_bias_of_another_form_keeps_its_route(form):
 
 @pytest.mark.parametrize("k,n,rows,K,cb,packed", [
     (4096, 6144, 560, 8, 0, False), (4096, 6144, 300, 4, 2, True), (4096, 4096, 768, 8, 0, False), (4096, 14336, 512, 4, 2, True), (4096, 14336, 600, 8, 1, False),
-    (14336, 4096, 1000, 4, 2, True), (2048, 512, 1000, 8, 0, True), (2048, 512, 1023, 4, 2, True), (2048, 512, 1024, 4, 2, False)])
+    (14336, 4096, 1000, 4, 2, True), (2048, 512, 1000, 8, 0, True), (2048, 512, 1023, 4, 2, True), (2048, 512, 1024, 4, 2, False),
+    (2048, 2048, 1023, 6, 2, False), (2048, 2048, 768, 6, 2, True), (4096, 22016, 400, 4, 2, True), (5120, 27648, 600, 4, 2, True), (4096, 28672, 1000, 8, 0, False)])
 def test_route_follows_sizes_bits_and_codebook(k, n, rows, K, cb, packed):
     """The route with the fp16 weight matrix gives the bits of the forced one, the packed one does not; points where the two are at least 5 % apart, and the last row count."""
     from exllamav3_amd.linear import LinearEXL3
