@@ -3,6 +3,7 @@
 #include "exl3_api_internal.h"
 #include "exl3_dgemm.h"
 #include "exl3_dgemm_api.h"
+#include <atomic>
 #include <math.h>
 #include <stdlib.h>
 #include <string.h>
@@ -185,12 +186,13 @@ static DgPlan dg_plan(int m, int k, int n, int K, int cb, int cus, int64_t max_f
 
 static int dg_device_cus(int* cus)
 {
-    static int cached[64] = { 0 };                        // (a property of the device; concurrent writers store the same value)
+    static std::atomic<int> cached[64];                   // (a property of the device; several threads store the same value)
     int dev = 0;
     EXL3_CHECK_HIP(hipGetDevice(&dev), "exl3_dgemm");
-    if (dev >= 0 && dev < 64 && cached[dev]) { *cus = cached[dev]; return EXL3_OK; }
+    const bool known = dev >= 0 && dev < 64;
+    if (known && (*cus = cached[dev].load(std::memory_order_relaxed)) != 0) return EXL3_OK;
     EXL3_CHECK_HIP(hipDeviceGetAttribute(cus, hipDeviceAttributeMultiprocessorCount, dev), "exl3_dgemm");
-    if (dev >= 0 && dev < 64) cached[dev] = *cus;
+    if (known) cached[dev].store(*cus, std::memory_order_relaxed);
     return EXL3_OK;
 }
 
