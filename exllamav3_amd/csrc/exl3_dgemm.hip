@@ -135,7 +135,10 @@ static DgKind dg_kind(int K, int cb)
 // slower than the best of the launches on average up to 128 rows (7 % at most) and 0.9 % above (13 %); without the terms of dg_kind they were 1.0 % (30 %) and 5.2 % (48 %) slower:
 // 8192 x 8192, 8 bits, 420 rows 134 us, 84 now.
 // Up to 128 rows (one row tile): a workgroup pays its prologue and epilogue once and `step` per 128 k.  Above: a wide workgroup has its CU alone, a last round that fills the chip in part runs
-// faster than a full one; two narrow workgroups share a CU at about the cost of one after the other.  A split writes and reads its partial sums and launches their reduction.
+// faster than a full one; two narrow workgroups share a CU at about the cost of one after the other.  A split writes and reads its partial sums and launches their reduction:
+// above 128 rows priced as in a stream, where that kernel follows without a gap (the launches were timed in graphs, whose next node costs 3 us more; and the sums of a wide kernel's eight slices
+// take 9 us to add where four slices take 6).  Over 2 463 launches with cold weights, less that gap, the choices are 1.1 % slower than the best on average as before, 11 % at most (19); chunks of
+// 180 .. 256 rows through four layers of 4096 / 14336: 4 % faster.
 static double dg_cost(const DgKind& kind, int m, int k, int n, int mt, int mtiles, int s, int b, int cus)
 {
     const double wgs = (double) mtiles * (n >> 7) * s;
@@ -148,11 +151,11 @@ static double dg_cost(const DgKind& kind, int m, int k, int n, int mt, int mtile
     if (mt > 8)
     {
         const double rounds = ceil(wgs / cus), last = wgs / cus - (rounds - 1.0);
-        return (rounds - 1.0 + 0.86 + 0.14 * last) * (b * (0.156 + kind.wide + 0.081 * mt) + 0.69 * mt) + (s > 1 ? 2.2 + 0.27 * sums + 0.10 * s : 0.0);
+        return (rounds - 1.0 + 0.86 + 0.14 * last) * (b * (0.156 + kind.wide + 0.081 * mt) + 0.69 * mt) + (s > 1 ? 0.5 * sums + 0.10 * s : 0.0);
     }
     const double one = b * (0.215 + kind.one + 0.112 * mt + 0.487 * deep) + 0.03 * mt, two = b * (0.828 + kind.two + 0.122 * mt) + 0.73 * mt;
     const double rounds = ceil(wgs / (2.0 * cus)), left = wgs - (rounds - 1.0) * 2.0 * cus;
-    return (rounds - 1.0) * two + (left > cus ? two * (0.50 + 0.50 * left / (2.0 * cus)) : one) + (s > 1 ? 3.4 + 0.36 * sums + 0.35 * s : 0.0);
+    return (rounds - 1.0) * two + (left > cus ? two * (0.50 + 0.50 * left / (2.0 * cus)) : one) + (s > 1 ? 1.0 + 0.36 * sums + 0.35 * s : 0.0);
 }
 
 // The cheapest kernel, row tiling and split whose partial sums fit max_floats
@@ -249,7 +252,8 @@ extern "C" int exl3_dgemm_pays(int m, int k, int n, int K, int cb)
     const int rc = dg_device_cus(&cus);
     if (rc != EXL3_OK) return rc;
     const double kn = 1e-6 * (double) k * n, tiles = (m + 255) / 256;
-    const double here = fmax(16.5, 9.5 + 1.243 * dg_plan(m, k, n, K, cb, cus, INT64_MAX).us);
+    const DgPlan plan = dg_plan(m, k, n, K, cb, cus, INT64_MAX);
+    const double here = fmax(16.5, 9.5 + 1.243 * (plan.us + (plan.S > 1 ? 2.3 : 0.0)));      // (2.3: the gap in front of the reduction, which the tiling is not charged for)
     // (30.5: the host's time for that route's launches, which is what small calls one after the other take; behind a queue of other work they take their device time, 1024 x 1024 at 1000 rows 21 us here
     // and 16 there, 2048 x 2048 29 and 26.  Many rows are such a queue: beyond 768 of them the device's time decides, but for long contractions)
     const double there = fmax(m > 768 && k < 2 * n ? 0.0 : 30.5, 15.3 + 0.669 * kn + 0.126 * kn * tiles + 0.616e-3 * kn * m + 0.88e-3 * k + 1.365e-6 * (double) k * m);
